@@ -4,8 +4,10 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <map>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "acc_cn.h"
@@ -39,7 +41,33 @@ struct CopyLane {
   hipEvent_t ev[2] = {nullptr, nullptr};
 };
 
+// Device memory of a context's graphs and workspaces.  Freed blocks are kept
+// for the next allocation of their size (up to an eighth and 64 KiB larger),
+// at most kPoolBytes of them, the largest going back to the device first;
+// all go back when an allocation fails and when the context ends.  A
+// hipMalloc and a hipFree take 30 and 40 us, and an upload with a SCAN query
+// made some 40 of each: 2.8 of its 7.6 ms at 262,144 vertices and 7.3M slots.
+// A block is reused without waiting: whoever frees one has waited for the
+// work that uses it, or that work and every later use are ordered by the
+// context's stream.  Safe from several threads.
+class DevicePool {
+ public:
+  hipError_t alloc(void **p, size_t bytes);
+  void free(void *p);
+  void trim();
+  ~DevicePool() { trim(); }
+
+ private:
+  void give_back(size_t most);  // with mu_ held
+  static constexpr size_t kPoolBytes = size_t(4) << 30;
+  std::mutex mu_;
+  std::multimap<size_t, void *> idle_;
+  std::unordered_map<void *, size_t> size_;  // of every block, idle or not
+  size_t idle_bytes_ = 0;
+};
+
 struct acc_ctx {
+  DevicePool pool;
   int device = 0;
   hipStream_t stream = nullptr;
   int num_cus = 0;
@@ -227,6 +255,7 @@ struct ScanBuffers {
   uint32_t n_cap = 0;
   uint64_t m_cap = 0;
   uint64_t bytes = 0;
+  DevicePool *pool = nullptr;  // where the buffers come from (NULL: hipMalloc)
 };
 
 namespace accscan {

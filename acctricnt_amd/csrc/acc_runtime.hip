@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <iterator>
 #include <numeric>
 #include <thread>
 #include <new>
@@ -19,7 +20,7 @@ struct DeviceGuard {
 template <typename T>
 int dev_alloc(acc_graph *g, T **p, uint64_t count) {
   const size_t bytes = sizeof(T) * (count ? count : 1);
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(p), bytes);
+  hipError_t e = g->ctx->pool.alloc(reinterpret_cast<void **>(p), bytes);
   if (e != hipSuccess) {
     *p = nullptr;
     return acc_set_error(ACC_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
@@ -32,6 +33,7 @@ int dev_alloc(acc_graph *g, T **p, uint64_t count) {
 void free_graph(acc_graph *g) {
   if (!g) return;
   DeviceGuard guard(g->ctx->device);
+  (void)hipDeviceSynchronize();  // queries on other streams may still read the graph
   for (void *p : {static_cast<void *>(g->d_off), static_cast<void *>(g->d_adj), static_cast<void *>(g->d_cnt),
                   static_cast<void *>(g->d_rev), static_cast<void *>(g->d_sum), static_cast<void *>(g->d_flags),
                   static_cast<void *>(g->d_fwd_wave), static_cast<void *>(g->d_fwd_block),
@@ -42,13 +44,11 @@ void free_graph(acc_graph *g) {
                   static_cast<void *>(g->edge.d_units[kEdgeHub]), static_cast<void *>(g->edge.d_hubs),
                   static_cast<void *>(g->edge.d_pool), static_cast<void *>(g->d_skey),
                   static_cast<void *>(g->d_snbr), static_cast<void *>(g->d_sslot),
-                  static_cast<void *>(g->d_tri_parts), static_cast<void *>(g->d_hs)})
-    if (p) (void)hipFree(p);
+                  static_cast<void *>(g->d_tri_parts), static_cast<void *>(g->d_hs),
+                  static_cast<void *>(g->d_gvoff), static_cast<void *>(g->d_gsoff), static_cast<void *>(g->d_gtot)})
+    g->ctx->pool.free(p);
   if (g->graph_exec) (void)hipGraphExecDestroy(g->graph_exec);
   if (g->graph) (void)hipGraphDestroy(g->graph);
-  if (g->d_gvoff) (void)hipFree(g->d_gvoff);
-  if (g->d_gsoff) (void)hipFree(g->d_gsoff);
-  if (g->d_gtot) (void)hipFree(g->d_gtot);
   for (hipEvent_t e : g->events) (void)hipEventDestroy(e);
   delete g;
 }
@@ -95,7 +95,7 @@ void build_edge_plan(uint32_t n, const uint32_t *off, const uint32_t *hs, uint32
 template <typename T>
 void dev_free(acc_graph *g, T **p, uint64_t count) {
   if (*p) {
-    (void)hipFree(*p);
+    g->ctx->pool.free(*p);
     g->device_bytes -= sizeof(T) * (count ? count : 1);
   }
   *p = nullptr;
@@ -351,7 +351,7 @@ int load_vertex_meta(acc_graph *g, const uint32_t *host_off) {
   const uint32_t n = g->n;
   ACC_TRY(dev_alloc(g, &g->d_hs, static_cast<uint64_t>(n) + 1));
   int32_t *lo = nullptr;
-  if (hipMalloc(reinterpret_cast<void **>(&lo), sizeof(int32_t) * (static_cast<size_t>(n) + 2)) != hipSuccess)
+  if (g->ctx->pool.alloc(reinterpret_cast<void **>(&lo), sizeof(int32_t) * (static_cast<size_t>(n) + 2)) != hipSuccess)
     return acc_set_error(ACC_ENOMEM, "hipMalloc of the vertex metadata failed");
   uint32_t *d_max = reinterpret_cast<uint32_t *>(lo + n);
   uint32_t h_max[2] = {0, 0};
@@ -370,7 +370,7 @@ int load_vertex_meta(acc_graph *g, const uint32_t *host_off) {
   if (!rc) rc = staged_copy(g->ctx, g->h_lo.data(), lo, sizeof(int32_t) * n, false);
   if (!rc) rc = staged_copy(g->ctx, h_max, d_max, sizeof(h_max), false);
   (void)hipStreamSynchronize(st);
-  (void)hipFree(lo);
+  g->ctx->pool.free(lo);
   if (rc) return rc;
   g->max_low = h_max[0];
   g->max_deg = h_max[1];
@@ -384,6 +384,55 @@ int record_event(acc_graph *g, const char *name) {
   const int rc = record(g, true, name);
   if (!rc && g->events.size() > 1) g->timing_valid = true;
   return rc;
+}
+
+hipError_t DevicePool::alloc(void **p, size_t bytes) {
+  *p = nullptr;
+  const size_t step = bytes > (size_t(1) << 20) ? size_t(64) << 10 : size_t(4) << 10;
+  bytes = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+  std::lock_guard<std::mutex> lk(mu_);
+  const auto it = idle_.lower_bound(bytes);
+  if (it != idle_.end() && it->first <= bytes + bytes / 8 + (size_t(64) << 10)) {
+    *p = it->second;
+    idle_bytes_ -= it->first;
+    idle_.erase(it);
+    return hipSuccess;
+  }
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && idle_bytes_) {
+    (void)hipGetLastError();
+    give_back(0);
+    e = hipMalloc(p, bytes);
+  }
+  if (e == hipSuccess)
+    size_[*p] = bytes;
+  else
+    *p = nullptr;
+  return e;
+}
+
+void DevicePool::free(void *p) {
+  if (!p) return;
+  std::lock_guard<std::mutex> lk(mu_);
+  const size_t bytes = size_[p];
+  idle_.emplace(bytes, p);
+  idle_bytes_ += bytes;
+  give_back(kPoolBytes);
+}
+
+void DevicePool::trim() {
+  std::lock_guard<std::mutex> lk(mu_);
+  give_back(0);
+}
+
+void DevicePool::give_back(size_t most) {
+  while (idle_bytes_ > most) {
+    const auto last = std::prev(idle_.end());
+    idle_bytes_ -= last->first;
+    size_.erase(last->second);
+    (void)hipFree(last->second);
+    idle_.erase(last);
+  }
 }
 
 int acc_set_error(int code, const std::string &msg) {
@@ -455,6 +504,7 @@ void acc_ctx_destroy(acc_ctx *ctx) {
       if (l.ev[b]) (void)hipEventDestroy(l.ev[b]);
     }
   }
+  ctx->pool.trim();
   delete ctx;
 }
 
@@ -844,7 +894,7 @@ int acc_graph_set_shard(acc_graph *g, uint32_t parts, uint32_t index, uint32_t *
       ACC_TRY(accfwd::launch_count(g));
       if (g->n_fwd_big) ACC_TRY(accfwd::launch_count_big(g));
       unsigned long long *d_work = nullptr;
-      ACC_HIP_TRY(hipMalloc(reinterpret_cast<void **>(&d_work), sizeof(unsigned long long) * n));
+      ACC_HIP_TRY(g->ctx->pool.alloc(reinterpret_cast<void **>(&d_work), sizeof(unsigned long long) * n));
       std::vector<unsigned long long> w(n);
       int rc = accfwd::launch_source_work(g, d_work);
       hipError_t e = hipSuccess;
@@ -852,7 +902,7 @@ int acc_graph_set_shard(acc_graph *g, uint32_t parts, uint32_t index, uint32_t *
                                   g->ctx->stream);
       if (!rc && e == hipSuccess) e = hipStreamSynchronize(g->ctx->stream);
       (void)hipStreamSynchronize(g->ctx->stream);
-      (void)hipFree(d_work);
+      g->ctx->pool.free(d_work);
       if (rc) return rc;
       if (e != hipSuccess) return acc_set_error(ACC_EDEVICE, std::string("source work: ") + hipGetErrorString(e));
       g->h_work.assign(static_cast<size_t>(n) + 1, 0);

@@ -738,25 +738,25 @@ int build_index(acc_graph *g) {
   size_t temp_bytes = 0;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(st);
-    if (key_in) (void)hipFree(key_in);
-    if (temp) (void)hipFree(temp);
+    g->ctx->pool.free(key_in);
+    g->ctx->pool.free(temp);
   };
   auto fail = [&](const char *what, hipError_t e) {
     cleanup();
     for (void **p : {reinterpret_cast<void **>(&g->d_skey), reinterpret_cast<void **>(&g->d_snbr),
                      reinterpret_cast<void **>(&g->d_sslot)})
       if (*p) {
-        (void)hipFree(*p);
+        g->ctx->pool.free(*p);
         *p = nullptr;
       }
     return acc_set_error(e == hipErrorOutOfMemory ? ACC_ENOMEM : ACC_EDEVICE,
                          std::string(what) + ": " + hipGetErrorString(e));
   };
   const size_t mm = m ? m : 1;
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(&key_in), sizeof(float) * mm);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&g->d_skey), sizeof(float) * mm);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&g->d_sslot), sizeof(uint32_t) * mm);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&g->d_snbr), sizeof(int32_t) * mm);
+  hipError_t e = g->ctx->pool.alloc(reinterpret_cast<void **>(&key_in), sizeof(float) * mm);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_skey), sizeof(float) * mm);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_sslot), sizeof(uint32_t) * mm);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_snbr), sizeof(int32_t) * mm);
   if (e != hipSuccess) return fail("index allocation", e);
   if (m) {
     // the sort is double-buffered (keys between key_in and d_skey, slots
@@ -772,7 +772,7 @@ int build_index(acc_graph *g) {
     e = hipcub::DeviceSegmentedRadixSort::SortPairsDescending(nullptr, temp_bytes, kb, sb, static_cast<int>(m),
                                                               static_cast<int>(g->n), g->d_off, g->d_off + 1, 0,
                                                               32, st);
-    if (e == hipSuccess) e = hipMalloc(&temp, temp_bytes ? temp_bytes : 1);
+    if (e == hipSuccess) e = g->ctx->pool.alloc(&temp, temp_bytes ? temp_bytes : 1);
     kb = hipcub::DoubleBuffer<float>(key_in, g->d_skey);  // as before the size query
     sb = hipcub::DoubleBuffer<uint32_t>(slot_in, g->d_sslot);
     if (e == hipSuccess)
@@ -822,7 +822,7 @@ void free_ws(acc_scan_ws *w) {
   (void)hipSetDevice(w->g->ctx->device);
   if (w->stream) (void)hipStreamSynchronize(w->stream);
   accscan::free_buffers(&w->buf);
-  if (w->d_pairs) (void)hipFree(w->d_pairs);
+  w->g->ctx->pool.free(w->d_pairs);
   if (w->ready) (void)hipEventDestroy(w->ready);
   if (w->stream) (void)hipStreamDestroy(w->stream);
   delete w;
@@ -838,8 +838,13 @@ void free_buffers(ScanBuffers *b) {
                   static_cast<void *>(b->label),
                   static_cast<void *>(b->parent), static_cast<void *>(b->rmin), static_cast<void *>(b->rmax),
                   static_cast<void *>(b->cl), static_cast<void *>(b->cid), static_cast<void *>(b->counters)})
-    if (p) (void)hipFree(p);
+    if (b->pool)
+      b->pool->free(p);
+    else if (p)
+      (void)hipFree(p);
+  DevicePool *const pool = b->pool;
   *b = ScanBuffers{};
+  b->pool = pool;
 }
 
 // Grows the per-query buffers to hold a graph of n vertices and m slots.
@@ -851,7 +856,8 @@ int reserve_buffers(ScanBuffers *b, uint32_t n, uint64_t m) {
   auto alloc = [&](auto **p, uint64_t count) -> int {
     using T = std::remove_pointer_t<std::remove_reference_t<decltype(*p)>>;
     const size_t bytes = sizeof(T) * (count ? count : 1);
-    if (hipMalloc(reinterpret_cast<void **>(p), bytes) != hipSuccess) {
+    void **const to = reinterpret_cast<void **>(p);
+    if ((b->pool ? b->pool->alloc(to, bytes) : hipMalloc(to, bytes)) != hipSuccess) {
       *p = nullptr;
       return acc_set_error(ACC_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes of SCAN buffers failed");
     }
@@ -927,7 +933,7 @@ ScanJob make_job(const acc_graph *g, const ScanBuffers &b, int64_t eps_num, int6
 // Builds the slot -> source array of a resident graph once.
 int acc_graph_ensure_src(acc_graph *g) {
   if (g->d_src) return ACC_OK;
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(&g->d_src), sizeof(int32_t) * (g->m ? g->m : 1));
+  hipError_t e = g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_src), sizeof(int32_t) * (g->m ? g->m : 1));
   if (e != hipSuccess) {
     g->d_src = nullptr;
     return acc_set_error(ACC_ENOMEM, "hipMalloc of the slot source array failed");
@@ -946,7 +952,8 @@ int acc_graph_set_vertex_ids(acc_graph *g, const int32_t *old_id) {
   (void)hipSetDevice(g->ctx->device);
   if (!old_id) {
     if (g->d_old) {
-      (void)hipFree(g->d_old);
+      ACC_HIP_TRY(hipDeviceSynchronize());  // queries on other streams may still read the ids
+      g->ctx->pool.free(g->d_old);
       g->device_bytes -= sizeof(int32_t) * (g->n ? g->n : 1);
     }
     g->d_old = nullptr;
@@ -955,7 +962,7 @@ int acc_graph_set_vertex_ids(acc_graph *g, const int32_t *old_id) {
   for (uint32_t u = 0; u < g->n; u++)
     if (old_id[u] < 0) return acc_set_error(ACC_EINVAL, "vertex ids must be non-negative");
   if (!g->d_old) {
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&g->d_old), sizeof(int32_t) * (g->n ? g->n : 1));
+    hipError_t e = g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_old), sizeof(int32_t) * (g->n ? g->n : 1));
     if (e != hipSuccess) {
       g->d_old = nullptr;
       return acc_set_error(ACC_ENOMEM, "hipMalloc of the vertex id array failed");
@@ -983,6 +990,7 @@ int acc_scan_ws_create(acc_graph *g, acc_scan_ws **out) {
   if (e != hipSuccess) return bail(acc_set_error(ACC_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e)));
   e = hipEventCreateWithFlags(&w->ready, hipEventDisableTiming);
   if (e != hipSuccess) return bail(acc_set_error(ACC_EDEVICE, std::string("hipEventCreate: ") + hipGetErrorString(e)));
+  w->buf.pool = &g->ctx->pool;
   if ((rc = accscan::reserve_buffers(&w->buf, g->n, g->m))) return bail(rc);
   w->device_bytes = w->buf.bytes;
   if ((rc = acc_graph_ensure_src(g))) return bail(rc);
@@ -1062,7 +1070,7 @@ int acc_scan_pairs(acc_scan_ws *w, int32_t *pairs, uint64_t cap, uint64_t *count
   // every slot is at most one pair: size the buffer for m once
   if (!w->d_pairs) {
     const size_t bytes = sizeof(int2) * (g->m ? g->m : 1);
-    if (hipMalloc(reinterpret_cast<void **>(&w->d_pairs), bytes) != hipSuccess) {
+    if (g->ctx->pool.alloc(reinterpret_cast<void **>(&w->d_pairs), bytes) != hipSuccess) {
       w->d_pairs = nullptr;
       return acc_set_error(ACC_ENOMEM, "hipMalloc of the pair buffer failed");
     }

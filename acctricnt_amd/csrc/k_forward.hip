@@ -1035,8 +1035,8 @@ int launch_count_big(acc_graph *g) { return launch_big_t<true>(g, nullptr); }
 
 int launch_triangles(acc_graph *g) {
   if (!g->d_tri_parts) {
-    if (hipMalloc(reinterpret_cast<void **>(&g->d_tri_parts), sizeof(unsigned long long) * kTriParts * kTriStride) !=
-        hipSuccess) {
+    if (g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_tri_parts),
+                           sizeof(unsigned long long) * kTriParts * kTriStride) != hipSuccess) {
       g->d_tri_parts = nullptr;
       return acc_set_error(ACC_ENOMEM, "hipMalloc of the triangle partial sums failed");
     }

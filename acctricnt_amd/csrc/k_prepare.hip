@@ -159,15 +159,14 @@ int slot_sources(acc_graph *g) {
   size_t t_bytes = 0;
   void *temp = nullptr;
   hipError_t e = hipcub::DeviceScan::InclusiveScan(nullptr, t_bytes, heads, src, hipcub::Max(), m, st);
-  if (e == hipSuccess) e = hipMalloc(&temp, t_bytes ? t_bytes : 1);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(&temp, t_bytes ? t_bytes : 1);
   if (e == hipSuccess) e = hipMemsetAsync(heads, 0, sizeof(uint32_t) * m, st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_rl_heads, dim3(rl_grid(g->n, g->ctx->num_cus)), dim3(256), 0, st, g->d_off, g->n, heads);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipcub::DeviceScan::InclusiveScan(temp, t_bytes, heads, src, hipcub::Max(), m, st);
-  (void)hipStreamSynchronize(st);
-  if (temp) (void)hipFree(temp);
+  g->ctx->pool.free(temp);  // its next use comes later on the same stream
   if (e != hipSuccess)
     return acc_set_error(e == hipErrorOutOfMemory ? ACC_ENOMEM : ACC_EDEVICE,
                          std::string("slot sources: ") + hipGetErrorString(e));
@@ -183,10 +182,8 @@ int reverse_slots(acc_graph *g, bool validate, uint64_t *upper) {
   const int cus = g->ctx->num_cus;
   uint32_t *low = nullptr, *L = nullptr;
   void *temp = nullptr;
-  auto cleanup = [&]() {
-    (void)hipStreamSynchronize(st);
-    for (void *p : {static_cast<void *>(low), static_cast<void *>(L), temp})
-      if (p) (void)hipFree(p);
+  auto cleanup = [&]() {  // the scratch's next use comes later on the same stream
+    for (void *p : {static_cast<void *>(low), static_cast<void *>(L), temp}) g->ctx->pool.free(p);
   };
   auto fail = [&](const char *what, hipError_t e) {
     cleanup();
@@ -194,11 +191,11 @@ int reverse_slots(acc_graph *g, bool validate, uint64_t *upper) {
                          std::string("reverse slots ") + what + ": " + hipGetErrorString(e));
   };
   const size_t nb1 = sizeof(uint32_t) * (static_cast<size_t>(n) + 1);
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(&low), nb1);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&L), nb1);
+  hipError_t e = g->ctx->pool.alloc(reinterpret_cast<void **>(&low), nb1);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&L), nb1);
   size_t t_scan = 0;
   if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(nullptr, t_scan, low, L, static_cast<int>(n) + 1, st);
-  if (e == hipSuccess) e = hipMalloc(&temp, t_scan ? t_scan : 1);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(&temp, t_scan ? t_scan : 1);
   if (e != hipSuccess) return fail("allocation", e);
   hipLaunchKernelGGL(k_rev_low, dim3(rl_grid(static_cast<uint64_t>(n) + 1, cus)), dim3(256), 0, st, g->d_off,
                      g->d_hs, n, low);
@@ -231,9 +228,9 @@ int reverse_slots(acc_graph *g, bool validate, uint64_t *upper) {
   size_t t_sort = 0;
   e = hipcub::DeviceRadixSort::SortPairs(nullptr, t_sort, kb, vb, static_cast<int>(count), 0, bits, st);
   if (e == hipSuccess && t_sort > t_scan) {
-    (void)hipFree(temp);
+    g->ctx->pool.free(temp);
     temp = nullptr;
-    e = hipMalloc(&temp, t_sort);
+    e = g->ctx->pool.alloc(&temp, t_sort);
   }
   if (e != hipSuccess) return fail("sort storage", e);
   hipLaunchKernelGGL(k_rev_keys, dim3(rl_grid(m, cus)), dim3(256), 0, st, g->d_adj,
@@ -271,26 +268,25 @@ int relabel_degree(acc_graph *g) {
   uint32_t *deg = nullptr, *deg_sorted = nullptr, *len = nullptr, *new_off = nullptr;
   int32_t *id = nullptr, *old_of_new = nullptr, *new_of_old = nullptr;
   void *temp = nullptr;
-  auto cleanup = [&]() {
-    (void)hipStreamSynchronize(st);
+  auto cleanup = [&]() {  // as in reverse_slots
     for (void *p : {static_cast<void *>(deg), static_cast<void *>(deg_sorted), static_cast<void *>(len),
                     static_cast<void *>(new_off), static_cast<void *>(id), static_cast<void *>(new_of_old), temp})
-      if (p) (void)hipFree(p);
+      g->ctx->pool.free(p);
   };
   auto fail = [&](const char *what, hipError_t e) {
     cleanup();
-    if (old_of_new) (void)hipFree(old_of_new);
+    g->ctx->pool.free(old_of_new);
     return acc_set_error(e == hipErrorOutOfMemory ? ACC_ENOMEM : ACC_EDEVICE,
                          std::string("relabel ") + what + ": " + hipGetErrorString(e));
   };
   const size_t nb = sizeof(uint32_t) * n, nb1 = sizeof(uint32_t) * (static_cast<size_t>(n) + 1);
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(&deg), nb);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&deg_sorted), nb);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&id), nb);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&old_of_new), nb);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&new_of_old), nb);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&len), nb1);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&new_off), nb1);
+  hipError_t e = g->ctx->pool.alloc(reinterpret_cast<void **>(&deg), nb);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&deg_sorted), nb);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&id), nb);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&old_of_new), nb);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&new_of_old), nb);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&len), nb1);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(reinterpret_cast<void **>(&new_off), nb1);
   if (e != hipSuccess) return fail("allocation", e);
   // cub temp storage: the largest of the three primitives' needs.  d_cnt
   // holds the slot sources (slot_sources); the reverse-slot array is free
@@ -310,7 +306,7 @@ int relabel_degree(acc_graph *g) {
     e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, t_seg, lb, static_cast<int>(m), static_cast<int>(n),
                                                    new_off, new_off + 1, 0, bits, st);
   size_t t_bytes = std::max(t_sort, std::max(t_scan, t_seg));
-  if (e == hipSuccess) e = hipMalloc(&temp, t_bytes ? t_bytes : 1);
+  if (e == hipSuccess) e = g->ctx->pool.alloc(&temp, t_bytes ? t_bytes : 1);
   if (e != hipSuccess) return fail("temporary storage", e);
 
   // device time of each step, read back with acc_cn_timings
@@ -321,7 +317,7 @@ int relabel_degree(acc_graph *g) {
   int rc = record_event(g, "begin");
   if (rc) {
     cleanup();
-    (void)hipFree(old_of_new);
+    g->ctx->pool.free(old_of_new);
     return rc;
   }
   hipLaunchKernelGGL(k_rl_keys, dim3(rl_grid(n, cus)), dim3(256), 0, st, g->d_off, n, deg, id);
@@ -355,7 +351,7 @@ int relabel_degree(acc_graph *g) {
   if (e != hipSuccess) return fail("offsets copy", e);
   (void)record_event(g, "rl_copy_offsets");
   cleanup();
-  if (g->d_old) (void)hipFree(g->d_old);
+  if (g->d_old) g->ctx->pool.free(g->d_old);
   else g->device_bytes += nb;
   g->d_old = old_of_new;
   g->relabelled = true;
