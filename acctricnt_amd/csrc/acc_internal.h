@@ -113,6 +113,27 @@ struct EdgePlan {
 };
 constexpr uint32_t kEdgeHashMax = 1u << 14;  // largest d_u an LDS hash table holds
 
+// Dense sources of the forward path (k_dense.hip): graph k of the partition
+// (one graph without a partition) starts at vertex first[k] and its first
+// limit[k] vertices are its dense sources.
+struct DensePlan {
+  std::vector<uint32_t> first, limit;
+  uint32_t most = 0;              // largest limit
+  uint32_t max_low = 0;           // most lower neighbors of a dense source
+  FwdUnit *d_units = nullptr;     // units of the shard's dense sources; nlow = the graph's first vertex
+  uint32_t n_units = 0;
+  uint4 *d_vmeta = nullptr;       // per vertex: first slot, first low group, hit base, rows
+  uint4 *d_low = nullptr;         // low lists, groups of eight 16-bit ids
+  uint32_t *d_large = nullptr;    // vertices with large hit matrices, then (one allocation)
+  uint32_t *d_mid = nullptr;      // those with medium ones
+  uint32_t n_large = 0, n_mid = 0;
+  uint32_t hit_cap = 0;           // most rows of a matrix that is kept
+  uint64_t hit_bytes = 0;         // of all matrices
+  uint8_t *d_hits = nullptr;      // allocated at the first per-slot pass
+  uint64_t bytes = 0, hits_held = 0;
+  bool tables = false;            // d_vmeta, d_low and d_large match first and limit
+};
+
 struct acc_graph {
   acc_ctx *ctx = nullptr;
   uint32_t n = 0;
@@ -144,6 +165,10 @@ struct acc_graph {
   uint32_t n_fwd_block = 0;
   FwdUnit *d_fwd_big = nullptr;  // |N<(b)| beyond the LDS table: global-memory lookups
   uint32_t n_fwd_big = 0;
+  DensePlan dense;           // dense sources and their tables
+  bool symmetric = false;    // every slot has its reverse (checked when the reverse slots are built)
+  bool dense_off = false;    // plan no dense sources (the shard work estimate reads per-probe hits)
+  std::vector<uint32_t> h_gvoff;  // the partition's vertex offsets
   EdgePlan edge;  // per-edge plans, built at the first bitmap or merge pass
   uint64_t device_bytes = 0;
   // tuning parameters (acc_graph_set_param)
@@ -277,9 +302,32 @@ bool index_usable(const acc_graph *g, int64_t p, int64_t q);
 int launch_index_jobs(const JobTable &jt, uint32_t vblocks, uint32_t sblocks, hipStream_t s);
 }  // namespace accscan
 
+// Dense sources (k_dense.hip).
+namespace accdense {
+constexpr uint32_t kMaxRows = 4096;  // most rows of a hit matrix that is kept
+// The vertex records, low lists and matrix offsets for dense.first / limit.
+int build_tables(acc_graph *g);
+void free_tables(acc_graph *g);
+// What a pass needs, where the plan has dense units: the tables and, with
+// `slots`, the hit matrices (allocated once; zeroed where only a share's rows
+// are written).  Not under capture.
+int ensure(acc_graph *g, bool slots);
+int clear_hits(acc_graph *g);
+int launch_count(acc_graph *g);
+int launch_triangles(acc_graph *g, unsigned long long *total);
+// Adds the hit matrices' row and column sums to the lower slots.
+int launch_rows(acc_graph *g);
+}  // namespace accdense
+
 // Kernel launchers (k_forward.hip).
 namespace accfwd {
-int launch_init(acc_graph *g);
+// Partial triangle totals of the triangle-only pass: kTriParts counters one
+// 128-byte line apart, workgroup w adding into counter w mod kTriParts, so
+// the atomics of many small units do not queue on one address.
+constexpr int kTriParts = 256;
+constexpr int kTriStride = 16;  // unsigned long longs per 128-byte line
+// Every slot gets `fill`.
+int launch_init(acc_graph *g, int fill);
 // Slot-parallel over the sources in d_cnt (accprep::slot_sources).  With
 // validate, d_flags[0] gets flag 8 for an upper slot without reverse and
 // d_flags[2..3] (a uint64) the number of upper slots.
@@ -288,8 +336,9 @@ int launch_build_rev(acc_graph *g, bool validate);
 int launch_triangles(acc_graph *g);
 int launch_count(acc_graph *g);
 int launch_count_big(acc_graph *g);
-// Adds each upper slot and its reverse; with a partition, also the per-graph
-// totals (which launch_init zeroes).
+// Adds each upper slot and its reverse, or with dense sources copies the
+// reverse slot's complete count; with a partition, also the per-graph totals
+// (which launch_init zeroes).
 int launch_combine(acc_graph *g, int plus);
 int launch_graph_totals(acc_graph *g, int plus);
 // Slot-parallel over the sources in d_cnt (accprep::slot_sources).
@@ -310,8 +359,8 @@ int launch_source_work(acc_graph *g, unsigned long long *work);
 // degree (d_rev is its scratch) and keeps the old id of every new vertex in
 // d_old; the sources must be recomputed after it.  reverse_slots, given the
 // sources and d_hs, fills d_rev (d_cnt is its scratch) and returns the number
-// of upper slots; with validate, an upper slot without its reverse sets flag
-// 8 in d_flags, and a count other than m / 2 leaves d_rev unbuilt.
+// of upper slots; an upper slot without its reverse sets flag 8 in d_flags,
+// and with validate a count other than m / 2 leaves d_rev unbuilt.
 namespace accprep {
 int slot_sources(acc_graph *g);
 int relabel_degree(acc_graph *g);

@@ -95,6 +95,7 @@ class HipDevice final : public accserve::Device {
     if (!rc) rc = acc_cn_compute(g, ACC_PATH_AUTO, 0);
     if (!rc) rc = acc_graph_ensure_src(g);
     if (!rc) rc = acc_ctx_synchronize(ctx_);
+    if (!rc) accdense::free_tables(g);  // a served graph is not counted again
     // the index is an optimisation: queries it cannot decide use the per-slot kernels
     if (!rc && !no_index_ && accscan::build_index(g) == ACC_OK) rc = acc_ctx_synchronize(ctx_);
     if (rc) {

@@ -29,6 +29,8 @@ using accfwd::kTableBits;
 using accfwd::kBigWG;
 using accfwd::kWG;
 using accfwd::kWaves;
+using accfwd::kTriParts;
+using accfwd::kTriStride;
 
 __device__ __forceinline__ uint32_t hash_slot(int32_t a, int bits) {
   return (static_cast<uint32_t>(a) * 0x9E3779B1u) >> (32 - bits);
@@ -46,17 +48,17 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
   return v;
 }
 
-// Zeroes the counts, the triangle sum and the per-graph totals of a
-// partitioned graph (parts of them; gtot may be NULL when parts is 0).
-__global__ __launch_bounds__(256) void k_init(int32_t *__restrict__ cnt, uint64_t m,
+// Sets the counts to `fill` and clears the triangle sum and the per-graph totals
+// of a partitioned graph (parts of them; gtot may be NULL when parts is 0).
+__global__ __launch_bounds__(256) void k_init(int32_t *__restrict__ cnt, uint64_t m, int fill,
                                               unsigned long long *__restrict__ sum,
                                               unsigned long long *__restrict__ gtot, uint32_t parts) {
   const uint64_t tid = blockIdx.x * 256ull + threadIdx.x;
   const uint64_t stride = gridDim.x * 256ull;
   const uint64_t m4 = m / 4;
-  const int4 z = make_int4(0, 0, 0, 0);
+  const int4 z = make_int4(fill, fill, fill, fill);
   for (uint64_t i = tid; i < m4; i += stride) reinterpret_cast<int4 *>(cnt)[i] = z;
-  for (uint64_t i = m4 * 4 + tid; i < m; i += stride) cnt[i] = 0;
+  for (uint64_t i = m4 * 4 + tid; i < m; i += stride) cnt[i] = fill;
   for (uint64_t k = tid; k < parts; k += stride) gtot[k] = 0;
   if (tid == 0) *sum = 0;
 }
@@ -273,6 +275,17 @@ struct BitSet {
   }
 };
 
+// The count of probe j, an upper slot (b, c): stored there for the combine
+// to add, or (to_lower) added to the reverse slot, which then collects the
+// edge's whole count.
+__device__ __forceinline__ void put_probe(int32_t *cnt, const uint32_t *__restrict__ rev, uint32_t j, int v,
+                                          bool to_lower) {
+  if (!to_lower)
+    cnt[j] = v;
+  else if (v)
+    atomicAdd(&cnt[rev[j]], v);
+}
+
 // Exclusive prefix sum of v over the 64 lanes of a wave.
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane) {
   uint32_t x = v;
@@ -320,11 +333,6 @@ __device__ __forceinline__ void count_round(int32_t *reg, int k, bool hit, int l
   }
 }
 
-// Partial triangle totals of the triangle-only pass: kTriParts counters one
-// 128-byte line apart, workgroup w adding into counter w mod kTriParts, so
-// the atomics of many small units do not queue on one address.
-constexpr int kTriParts = 256;
-constexpr int kTriStride = 16;  // unsigned long longs per 128-byte line
 __device__ __forceinline__ unsigned long long *tri_part(unsigned long long *parts) {
   return parts + (blockIdx.x % kTriParts) * kTriStride;
 }
@@ -421,7 +429,7 @@ __device__ __forceinline__ uint32_t block_probe_flat(const int32_t *__restrict__
 // kSlots false: count the unit's triangles into *total instead of writing slots.
 template <int U, bool kSlots>
 __device__ __forceinline__ void fwd_block_unit(const uint32_t *__restrict__ off, const int32_t *__restrict__ adj,
-                                               const uint32_t *__restrict__ rev, const FwdUnit u, int32_t *cnt,
+                                               const uint32_t *__restrict__ rev, const FwdUnit u, bool to_lower, int32_t *cnt,
                                                unsigned long long *total, unsigned char *smem) {
   int32_t *keys = reinterpret_cast<int32_t *>(smem);  // hash keys, or bitmap words
   int32_t *ctr = keys + kBT;
@@ -495,7 +503,7 @@ __device__ __forceinline__ void fwd_block_unit(const uint32_t *__restrict__ off,
     return;
   }
   __syncthreads();
-  if (static_cast<uint32_t>(tid) < nup) cnt[u.j0 + tid] = s_reg[tid];
+  if (static_cast<uint32_t>(tid) < nup) put_probe(cnt, rev, u.j0 + tid, s_reg[tid], to_lower);
   for (uint32_t i = tid; i < nctr; i += kWG) {
     const int v = ctr[i];
     if (v) atomicAdd(&cnt[sb + i], v);
@@ -531,8 +539,8 @@ __device__ __forceinline__ int pack_bits(uint32_t nl) {
 template <int U, bool kSlots>
 __device__ __forceinline__ void fwd_pack_unit(const uint32_t *__restrict__ off, const uint32_t *__restrict__ hs,
                                               const int32_t *__restrict__ adj, const uint32_t *__restrict__ rev,
-                                              const FwdUnit u, int32_t *cnt, unsigned long long *total,
-                                              unsigned char *smem, int wave) {
+                                              const FwdUnit u, bool to_lower, int32_t *cnt,
+                                              unsigned long long *total, unsigned char *smem, int wave) {
   int32_t *base = reinterpret_cast<int32_t *>(smem);
   int32_t *keys = base + wave * kWT;
   int32_t *ctr = base + kWaves * kWT + wave * accfwd::kWaveCap;
@@ -674,7 +682,7 @@ __device__ __forceinline__ void fwd_pack_unit(const uint32_t *__restrict__ off, 
     return;
   }
   wave_lds_sync();
-  if (probe) cnt[j] = reg[lane];
+  if (probe) put_probe(cnt, rev, j, reg[lane], to_lower);
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const uint32_t e = lane + 64u * r;
@@ -704,18 +712,18 @@ __global__ __launch_bounds__(kWG) void k_fwd_count(const uint32_t *__restrict__ 
                                                    const uint32_t *__restrict__ rev,
                                                    const FwdUnit *__restrict__ block_units, uint32_t n_block,
                                                    const FwdUnit *__restrict__ wave_units, uint32_t n_wave,
-                                                   int32_t *cnt, unsigned long long *total) {
+                                                   bool to_lower, int32_t *cnt, unsigned long long *total) {
   __shared__ __align__(16) unsigned char smem[kCountLdsBytes];
   const uint32_t tasks = n_block + (n_wave + kWaves - 1) / kWaves;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t t = blockIdx.x;
   for (; t < n_block; t += gridDim.x) {
-    fwd_block_unit<U, kSlots>(off, adj, rev, block_units[t], cnt, total, smem);
+    fwd_block_unit<U, kSlots>(off, adj, rev, block_units[t], to_lower, cnt, total, smem);
     __syncthreads();
   }
   for (; t < tasks; t += gridDim.x) {
     const uint32_t ui = (t - n_block) * kWaves + wave;
-    if (ui < n_wave) fwd_pack_unit<U, kSlots>(off, hs, adj, rev, wave_units[ui], cnt, total, smem, wave);
+    if (ui < n_wave) fwd_pack_unit<U, kSlots>(off, hs, adj, rev, wave_units[ui], to_lower, cnt, total, smem, wave);
   }
 }
 
@@ -726,8 +734,8 @@ template <bool kSlots>
 __global__ __launch_bounds__(accfwd::kBigWG) void k_fwd_big(const uint32_t *__restrict__ off,
                                                             const int32_t *__restrict__ adj,
                                                             const uint32_t *__restrict__ rev,
-                                                            const FwdUnit *__restrict__ units, int32_t *cnt,
-                                                            unsigned long long *total) {
+                                                            const FwdUnit *__restrict__ units, bool to_lower,
+                                                            int32_t *cnt, unsigned long long *total) {
   const FwdUnit u = units[blockIdx.x];
   const int32_t b = u.b;
   const uint32_t sb = off[b];
@@ -764,13 +772,30 @@ __global__ __launch_bounds__(accfwd::kBigWG) void k_fwd_big(const uint32_t *__re
     reg = wave_sum_i32(reg);
     if (lane == 0) {
       if (kSlots)
-        cnt[j] = reg;
+        put_probe(cnt, rev, j, reg, to_lower);
       else if (reg)
         atomicAdd(tri_part(total), static_cast<unsigned long long>(reg));
     }
   }
 }
 
+// The count of the edge whose upper slot is i and lower slot p, written to
+// both; returns the raw count.  kGather: the lower slot holds it already, plus
+// included, and only the upper slot is written.
+template <bool kGather>
+__device__ __forceinline__ int combine_edge(int32_t *__restrict__ cnt, uint64_t i, uint32_t p, int plus) {
+  if (kGather) {
+    const int c = cnt[p];
+    cnt[i] = c;
+    return c - plus;
+  }
+  const int c = cnt[i] + cnt[p];
+  cnt[i] = c + plus;
+  cnt[p] = c + plus;
+  return c;
+}
+
+template <bool kGather>
 __global__ __launch_bounds__(256) void k_combine(int32_t *__restrict__ cnt, const uint32_t *__restrict__ rev,
                                                  uint64_t m, int plus, unsigned long long *__restrict__ sum) {
   __shared__ unsigned long long part[4];
@@ -779,13 +804,7 @@ __global__ __launch_bounds__(256) void k_combine(int32_t *__restrict__ cnt, cons
   unsigned long long s = 0;
   for (uint64_t i = tid; i < m; i += stride) {
     const uint32_t p = rev[i];
-    if (p < m) {
-      int c = cnt[i] + cnt[p];
-      s += static_cast<unsigned long long>(c);
-      c += plus;
-      cnt[i] = c;
-      cnt[p] = c;
-    }
+    if (p < m) s += static_cast<unsigned long long>(combine_edge<kGather>(cnt, i, p, plus));
   }
   s = wave_sum_u64(s);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
@@ -880,6 +899,7 @@ __device__ __forceinline__ uint32_t xcd_span(uint32_t b, uint32_t N) {
 // boundaries (a reverse slot lies in its upper slot's graph), combines every
 // upper slot of a piece and adds twice the piece's raw edge totals (both
 // slots of every edge: 6 T_k in all) to its graph's total.
+template <bool kGather>
 __global__ __launch_bounds__(256) void k_combine_parts(int32_t *__restrict__ cnt, const uint32_t *__restrict__ rev,
                                                        uint32_t m, int plus, unsigned long long *__restrict__ sum,
                                                        const uint32_t *__restrict__ gsoff, uint32_t parts,
@@ -901,13 +921,7 @@ __global__ __launch_bounds__(256) void k_combine_parts(int32_t *__restrict__ cnt
     unsigned long long s = 0;
     for (uint32_t i = s0 + threadIdx.x; i < e; i += 256) {
       const uint32_t p = rev[i];
-      if (p < m) {
-        int c = cnt[i] + cnt[p];
-        s += static_cast<unsigned long long>(c);
-        c += plus;
-        cnt[i] = c;
-        cnt[p] = c;
-      }
+      if (p < m) s += static_cast<unsigned long long>(combine_edge<kGather>(cnt, i, p, plus));
     }
     s = wave_sum_u64(s);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
@@ -957,9 +971,9 @@ inline unsigned grid_for(uint64_t items, int cus) {
 
 namespace accfwd {
 
-int launch_init(acc_graph *g) {
+int launch_init(acc_graph *g, int fill) {
   hipLaunchKernelGGL(k_init, dim3(grid_for(g->m / 4 + 1, g->ctx->num_cus)), dim3(256), 0, g->ctx->stream,
-                     g->d_cnt, g->m, g->d_sum, g->num_parts ? g->d_gtot : nullptr, g->num_parts);
+                     g->d_cnt, g->m, fill, g->d_sum, g->num_parts ? g->d_gtot : nullptr, g->num_parts);
   ACC_HIP_TRY(hipGetLastError());
   return ACC_OK;
 }
@@ -996,6 +1010,7 @@ int launch_vertex_meta(acc_graph *g, int32_t *lo, uint32_t *maxes) {
 template <bool kSlots>
 int launch_count_t(acc_graph *g, unsigned long long *total) {
   hipStream_t st = g->ctx->stream;
+  const bool to_lower = g->dense.n_units != 0;
   const uint64_t tasks = g->n_fwd_block + (g->n_fwd_wave + kWaves - 1) / kWaves;
   const uint64_t cap = static_cast<uint64_t>(g->persist) * static_cast<uint64_t>(g->ctx->num_cus);
   const unsigned grid = static_cast<unsigned>(g->persist && cap < tasks ? cap : tasks);
@@ -1003,15 +1018,15 @@ int launch_count_t(acc_graph *g, unsigned long long *total) {
     switch (g->fwd_unroll) {
       case 1:
         hipLaunchKernelGGL((k_fwd_count<1, kSlots>), dim3(grid), dim3(kWG), 0, st, g->d_off, g->d_hs, g->d_adj, g->d_rev,
-                           g->d_fwd_block, g->n_fwd_block, g->d_fwd_wave, g->n_fwd_wave, g->d_cnt, total);
+                           g->d_fwd_block, g->n_fwd_block, g->d_fwd_wave, g->n_fwd_wave, to_lower, g->d_cnt, total);
         break;
       case 4:
         hipLaunchKernelGGL((k_fwd_count<4, kSlots>), dim3(grid), dim3(kWG), 0, st, g->d_off, g->d_hs, g->d_adj, g->d_rev,
-                           g->d_fwd_block, g->n_fwd_block, g->d_fwd_wave, g->n_fwd_wave, g->d_cnt, total);
+                           g->d_fwd_block, g->n_fwd_block, g->d_fwd_wave, g->n_fwd_wave, to_lower, g->d_cnt, total);
         break;
       default:
         hipLaunchKernelGGL((k_fwd_count<2, kSlots>), dim3(grid), dim3(kWG), 0, st, g->d_off, g->d_hs, g->d_adj, g->d_rev,
-                           g->d_fwd_block, g->n_fwd_block, g->d_fwd_wave, g->n_fwd_wave, g->d_cnt, total);
+                           g->d_fwd_block, g->n_fwd_block, g->d_fwd_wave, g->n_fwd_wave, to_lower, g->d_cnt, total);
         break;
     }
     ACC_HIP_TRY(hipGetLastError());
@@ -1023,7 +1038,7 @@ template <bool kSlots>
 int launch_big_t(acc_graph *g, unsigned long long *total) {
   if (g->n_fwd_big) {
     hipLaunchKernelGGL(k_fwd_big<kSlots>, dim3(g->n_fwd_big), dim3(kBigWG), 0, g->ctx->stream, g->d_off, g->d_adj,
-                       g->d_rev, g->d_fwd_big, g->d_cnt, total);
+                       g->d_rev, g->d_fwd_big, g->dense.n_units != 0, g->d_cnt, total);
     ACC_HIP_TRY(hipGetLastError());
   }
   return ACC_OK;
@@ -1034,6 +1049,7 @@ int launch_count(acc_graph *g) { return launch_count_t<true>(g, nullptr); }
 int launch_count_big(acc_graph *g) { return launch_big_t<true>(g, nullptr); }
 
 int launch_triangles(acc_graph *g) {
+  ACC_TRY(accdense::ensure(g, false));
   if (!g->d_tri_parts) {
     if (g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_tri_parts),
                            sizeof(unsigned long long) * kTriParts * kTriStride) != hipSuccess) {
@@ -1045,6 +1061,7 @@ int launch_triangles(acc_graph *g) {
   hipStream_t st = g->ctx->stream;
   hipLaunchKernelGGL(k_tri_zero, dim3(1), dim3(kTriParts), 0, st, g->d_tri_parts);
   ACC_HIP_TRY(hipGetLastError());
+  ACC_TRY(accdense::launch_triangles(g, g->d_tri_parts));
   ACC_TRY(launch_count_t<false>(g, g->d_tri_parts));
   ACC_TRY(launch_big_t<false>(g, g->d_tri_parts));
   hipLaunchKernelGGL(k_tri_sum, dim3(1), dim3(kTriParts), 0, st, g->d_tri_parts, g->d_sum + 1);
@@ -1053,16 +1070,17 @@ int launch_triangles(acc_graph *g) {
 }
 
 int launch_combine(acc_graph *g, int plus) {
+  const bool gather = g->dense.n_units != 0;
   if (g->num_parts) {
     if (g->m) {
       const uint32_t blocks = static_cast<uint32_t>((g->m + kCombSpan - 1) / kCombSpan);
-      hipLaunchKernelGGL(k_combine_parts, dim3(blocks), dim3(256), 0, g->ctx->stream, g->d_cnt, g->d_rev,
+      hipLaunchKernelGGL((gather ? k_combine_parts<true> : k_combine_parts<false>), dim3(blocks), dim3(256), 0, g->ctx->stream, g->d_cnt, g->d_rev,
                          static_cast<uint32_t>(g->m), plus, g->d_sum, g->d_gsoff, g->num_parts, g->d_gtot);
     }
     ACC_HIP_TRY(hipGetLastError());
     return ACC_OK;
   }
-  hipLaunchKernelGGL(k_combine, dim3(grid_for(g->m, g->ctx->num_cus)), dim3(256), 0, g->ctx->stream, g->d_cnt,
+  hipLaunchKernelGGL((gather ? k_combine<true> : k_combine<false>), dim3(grid_for(g->m, g->ctx->num_cus)), dim3(256), 0, g->ctx->stream, g->d_cnt,
                      g->d_rev, g->m, plus, g->d_sum);
   ACC_HIP_TRY(hipGetLastError());
   return ACC_OK;

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256) void k_rev_fill(const uint32_t *__restrict__ k
     }
     if (!ok) f = 8;
   }
-  if (flags && f) atomicOr(flags, f);
+  if (f) atomicOr(flags, f);
 }
 
 unsigned rl_grid(uint64_t items, int cus) {
@@ -217,7 +217,7 @@ int reverse_slots(acc_graph *g, bool validate, uint64_t *upper) {
   // per-slot binary search instead.
   if (2 * count > m + 4 || count > static_cast<uint64_t>(INT32_MAX)) {
     cleanup();
-    return accfwd::launch_build_rev(g, false);
+    return accfwd::launch_build_rev(g, false);  // more upper than lower slots: not symmetric
   }
   uint32_t *keys_in = g->d_rev, *vals_in = g->d_rev + count;
   uint32_t *keys_out = reinterpret_cast<uint32_t *>(g->d_cnt), *vals_out = keys_out + count;
@@ -247,8 +247,7 @@ int reverse_slots(acc_graph *g, bool validate, uint64_t *upper) {
   if (e == hipSuccess) e = hipMemsetAsync(g->d_rev, 0xff, sizeof(uint32_t) * (m + 4), st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_rev_fill, dim3(rl_grid(count, cus)), dim3(256), 0, st, keys_out, vals_out,
-                       static_cast<uint32_t>(count), g->d_off, g->d_adj, L, n, g->d_rev,
-                       validate ? g->d_flags : nullptr);
+                       static_cast<uint32_t>(count), g->d_off, g->d_adj, L, n, g->d_rev, g->d_flags);
     e = hipGetLastError();
   }
   if (e != hipSuccess) return fail("build", e);
