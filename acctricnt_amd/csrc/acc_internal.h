@@ -167,7 +167,7 @@ struct acc_graph {
   uint32_t n_fwd_big = 0;
   DensePlan dense;           // dense sources and their tables
   bool symmetric = false;    // every slot has its reverse (checked when the reverse slots are built)
-  bool dense_off = false;    // plan no dense sources (the shard work estimate reads per-probe hits)
+  bool split_counts = false; // leave per-probe hits in the upper slots (the shard work estimate reads them)
   std::vector<uint32_t> h_gvoff;  // the partition's vertex offsets
   EdgePlan edge;  // per-edge plans, built at the first bitmap or merge pass
   uint64_t device_bytes = 0;
@@ -326,6 +326,11 @@ namespace accfwd {
 // the atomics of many small units do not queue on one address.
 constexpr int kTriParts = 256;
 constexpr int kTriStride = 16;  // unsigned long longs per 128-byte line
+// Whether a pass collects every edge's count in its lower slot, which the
+// combine copies to the upper one.  Otherwise (an upload trusted without
+// validation that is not symmetric, the shard work estimate) the upper slot holds
+// its probe's hits, the lower slot the rest, and the combine adds them.
+inline bool lower_counts(const acc_graph *g) { return g->symmetric && !g->split_counts; }
 // Every slot gets `fill`.
 int launch_init(acc_graph *g, int fill);
 // Slot-parallel over the sources in d_cnt (accprep::slot_sources).  With
@@ -336,9 +341,9 @@ int launch_build_rev(acc_graph *g, bool validate);
 int launch_triangles(acc_graph *g);
 int launch_count(acc_graph *g);
 int launch_count_big(acc_graph *g);
-// Adds each upper slot and its reverse, or with dense sources copies the
-// reverse slot's complete count; with a partition, also the per-graph totals
-// (which launch_init zeroes).
+// Copies the lower slots' counts to the upper ones or adds the two
+// (lower_counts); with a partition, also the per-graph totals (which
+// launch_init zeroes).
 int launch_combine(acc_graph *g, int plus);
 int launch_graph_totals(acc_graph *g, int plus);
 // Slot-parallel over the sources in d_cnt (accprep::slot_sources).

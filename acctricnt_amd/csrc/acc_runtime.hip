@@ -179,7 +179,7 @@ void plan_dense(acc_graph *g, std::vector<FwdUnit> &units, std::vector<SourceRan
   uint64_t upper = 0;
   for (size_t k = 0; k < first.size(); k++)
     limit.push_back(dense_sources(first[k], k + 1 < first.size() ? first[k + 1] : g->n, off, hs, &upper));
-  if (!g->symmetric || g->dense_off || upper < kDenseMin) std::fill(limit.begin(), limit.end(), 0u);
+  if (!accfwd::lower_counts(g) || upper < kDenseMin) std::fill(limit.begin(), limit.end(), 0u);
   for (size_t k = 0; k < first.size(); k++) {
     const uint32_t v0 = first[k];
     const uint32_t lo = std::max(v0, g->shard_lo), hi = std::min(v0 + limit[k], g->shard_hi);
@@ -706,10 +706,8 @@ int acc_cn_compute(acc_graph *g, int path, uint32_t flags) {
     g->timing_valid = timing;
     return ACC_OK;
   }
-  // With dense sources every edge's count collects in its lower slot, which
-  // starts at `plus`; otherwise in both of its slots.
-  const bool dense = g->dense.n_units != 0;
-  ACC_TRY(accfwd::launch_init(g, dense ? plus : 0));
+  // a lower slot that collects its edge's whole count starts at `plus`
+  ACC_TRY(accfwd::launch_init(g, accfwd::lower_counts(g) ? plus : 0));
   ACC_TRY(record(g, timing, "k_init"));
   ACC_TRY(accdense::launch_count(g));
   ACC_TRY(accfwd::launch_count(g));
@@ -718,7 +716,7 @@ int acc_cn_compute(acc_graph *g, int path, uint32_t flags) {
     ACC_TRY(accfwd::launch_count_big(g));
     ACC_TRY(record(g, timing, "k_fwd_big"));
   }
-  if (dense) {
+  if (g->dense.n_units) {
     ACC_TRY(accdense::launch_rows(g));
     ACC_TRY(record(g, timing, "k_dense_rows"));
   }
@@ -961,20 +959,20 @@ int acc_graph_set_shard(acc_graph *g, uint32_t parts, uint32_t index, uint32_t *
       // upper slot (b, c) its probe's hits, which the work estimate weighs
       g->shard_lo = 0;
       g->shard_hi = n;
-      g->dense_off = true;  // dense sources leave no hits in the upper slots
-      const int plan_rc = upload_plans(g);
-      g->dense_off = false;
-      ACC_TRY(plan_rc);
-      replan = true;
       g->have_result = false;
       g->totals_valid = false;
-      ACC_TRY(accfwd::launch_init(g, 0));
-      ACC_TRY(accfwd::launch_count(g));
-      if (g->n_fwd_big) ACC_TRY(accfwd::launch_count_big(g));
+      replan = true;
+      g->split_counts = true;
+      int rc = upload_plans(g);
+      if (!rc) rc = accfwd::launch_init(g, 0);
+      if (!rc) rc = accfwd::launch_count(g);
+      if (!rc && g->n_fwd_big) rc = accfwd::launch_count_big(g);
+      g->split_counts = false;
+      ACC_TRY(rc);
       unsigned long long *d_work = nullptr;
       ACC_HIP_TRY(g->ctx->pool.alloc(reinterpret_cast<void **>(&d_work), sizeof(unsigned long long) * n));
       std::vector<unsigned long long> w(n);
-      int rc = accfwd::launch_source_work(g, d_work);
+      rc = accfwd::launch_source_work(g, d_work);
       hipError_t e = hipSuccess;
       if (!rc) e = hipMemcpyAsync(w.data(), d_work, sizeof(unsigned long long) * n, hipMemcpyDeviceToHost,
                                   g->ctx->stream);
