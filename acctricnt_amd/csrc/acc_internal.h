@@ -251,6 +251,7 @@ struct ScanJob {
   uint32_t n;
   int32_t add;  // added to cnt to get 2 + |N(u) ∩ N(v)|
   int32_t mu;
+  uint32_t symmetric;  // every slot has its reverse (an upload trusted without validation may not)
   uint32_t vb0, vbn;  // workgroups of vertex-sized launches
   uint32_t sb0, sbn;  // workgroups of slot-sized launches
 };
