@@ -134,6 +134,8 @@ struct DensePlan {
   bool tables = false;            // d_vmeta, d_low and d_large match first and limit
 };
 
+constexpr uint32_t kAdjPad = 64;  // ids allocated past the adjacency array's end, 0
+
 struct acc_graph {
   acc_ctx *ctx = nullptr;
   uint32_t n = 0;
@@ -209,6 +211,9 @@ struct acc_graph {
 
 // Per-edge path launchers (k_paths.hip).
 namespace accpaths {
+// Graphs of at most this many vertices keep a hub's bitmap in LDS.
+constexpr uint32_t kLdsBitmapIds = 1u << 19;
+inline bool hubs_in_lds(const acc_graph *g) { return g->n <= kLdsBitmapIds; }
 int launch_bitmap(acc_graph *g, int plus);
 int launch_merge(acc_graph *g, int plus);
 }  // namespace accpaths

@@ -60,13 +60,14 @@ void free_graph(acc_graph *g) {
 // source), LDS hash classes of 2^12, 2^14 and 2^15 keys for d_u up to 2048,
 // 8192 and min(16384, hash_max); the rest are hubs.  Hubs go into batches of at
 // most pool_hubs (one HBM bitmap each); a hub unit's nlow is its hub's
-// bitmap within the batch.
+// bitmap within the batch.  Where hub bitmaps lie in LDS (lds_hubs), the
+// smallest block units, d_u <= 256, are hubs too.
 constexpr uint64_t kHubPoolBytes = 8ull << 30;  // HBM bitmaps of one hub batch
 constexpr uint32_t kHubBatch = 16384;           // most hubs of one batch (ACC_PARAM_BMP_BATCH)
 constexpr uint32_t kHashIdxBits = 1u << 17;     // LDS index bits of a hash unit (k_bmp_hash's kIdxWords)
 constexpr uint32_t kHubIdxBits = 1u << 18;      // LDS index bits of a hub unit (k_bmp_hub's kHubIdxWords)
 void build_edge_plan(uint32_t n, const uint32_t *off, const uint32_t *hs, uint32_t chunk, uint32_t hash_max,
-                     uint32_t pool_hubs, std::vector<FwdUnit> (&units)[kEdgeClasses], std::vector<uint32_t> &hubs,
+                     uint32_t pool_hubs, bool lds_hubs, std::vector<FwdUnit> (&units)[kEdgeClasses], std::vector<uint32_t> &hubs,
                      std::vector<uint32_t> &hub_batch, std::vector<uint32_t> &hub_unit_batch) {
   hub_batch.assign(1, 0);
   hub_unit_batch.assign(1, 0);
@@ -76,7 +77,7 @@ void build_edge_plan(uint32_t n, const uint32_t *off, const uint32_t *hs, uint32
     int c = kEdgeHub;
     if (du <= kEdgeWaveDeg && off[u + 1] - hs[u] <= kEdgeWaveUp)
       c = kEdgeWave;
-    else if (du <= hash_max)
+    else if (du <= hash_max && !(lds_hubs && du <= kEdgeWaveDeg))
       c = du <= 2048 ? kEdgeHash12 : du <= 8192 ? kEdgeHash14 : kEdgeHash15;
     uint32_t slot = 0;
     if (c == kEdgeHub) {
@@ -246,7 +247,7 @@ int ensure_edge_plans(acc_graph *g) {
       std::min<uint64_t>(g->bmp_batch, std::max<uint64_t>(1, kHubPoolBytes / (sizeof(uint32_t) * p.pool_words))));
   std::vector<FwdUnit> units[kEdgeClasses];
   std::vector<uint32_t> hubs;
-  build_edge_plan(g->n, g->h_off.data(), g->h_hs.data(), g->chunk, g->bmp_hash_max, pool_hubs, units, hubs,
+  build_edge_plan(g->n, g->h_off.data(), g->h_hs.data(), g->chunk, g->bmp_hash_max, pool_hubs, accpaths::hubs_in_lds(g), units, hubs,
                   p.hub_batch, p.hub_unit_batch);
   PlanList lists[] = {{&units[kEdgeWave], &p.d_units[kEdgeWave], &p.n_units[kEdgeWave]},
                       {&units[kEdgeHash12], &p.d_units[kEdgeHash12], &p.n_units[kEdgeHash12]},
@@ -269,6 +270,7 @@ int ensure_edge_plans(acc_graph *g) {
 // The hub bitmap pool (zeroed once: every bitmap pass clears what it sets).
 int ensure_bitmap_pool(acc_graph *g) {
   EdgePlan &p = g->edge;
+  if (accpaths::hubs_in_lds(g)) return ACC_OK;
   uint32_t need = 0;
   for (size_t k = 0; k + 1 < p.hub_batch.size(); k++) need = std::max(need, p.hub_batch[k + 1] - p.hub_batch[k]);
   if (need <= p.pool_hubs) return ACC_OK;
@@ -609,7 +611,7 @@ int acc_graph_upload(acc_ctx *ctx, uint32_t n, uint64_t m, const uint32_t *node_
     return code;
   };
   if ((rc = dev_alloc(g, &g->d_off, static_cast<uint64_t>(n) + 1))) return bail(rc);
-  if ((rc = dev_alloc(g, &g->d_adj, m + 64))) return bail(rc);
+  if ((rc = dev_alloc(g, &g->d_adj, m + kAdjPad))) return bail(rc);
   if ((rc = dev_alloc(g, &g->d_cnt, m + 4))) return bail(rc);
   if ((rc = dev_alloc(g, &g->d_rev, m + 4))) return bail(rc);
   if ((rc = dev_alloc(g, &g->d_sum, 2))) return bail(rc);

@@ -7,7 +7,8 @@
 //   neighbor list N(v), v > u, is probed against it.  Small sets (up to
 //   ACC_PARAM_BMP_HASH_MAX ids, 256 by default) live in an LDS hash table,
 //   behind an LDS index of N(u) (one bit per 32 ids) in a workgroup unit;
-//   larger sets spill to an n-bit bitmap in HBM,
+//   larger sets are an n-bit bitmap, in LDS up to 2^19 vertices (k_bmp_lds, for
+//   the small sets of workgroup units too) and beyond that in HBM,
 //   built for a batch of hubs by one kernel and shared by every workgroup
 //   that probes that hub, with an LDS index of one bit per 16 ids (per
 //   larger group beyond 2^18 groups) checked before the HBM word, the
@@ -36,6 +37,8 @@
 // slot (u, v) and its reverse slot (from the reverse-slot index built at
 // upload), with no atomics on the counts, and adds the raw counts to the
 // triangle sum.
+
+#include <algorithm>
 
 #include "acc_internal.h"
 #include "flat_window.h"
@@ -441,6 +444,159 @@ __global__ __launch_bounds__(kWG) void k_bmp_hub(const uint32_t *__restrict__ of
   finish_unit(L, rev, un.j0, nup, cnt, plus, sum);
 }
 
+// Hub units of a graph whose n-bit bitmap fits LDS (accpaths::kLdsBitmapIds):
+// the set of N(u) is that bitmap, id a at bit 31 - (a mod 32) of word a / 32
+// (a shift left by a's low bits leaves the membership in the sign bit).  The
+// probed lists are laid end to end in groups of four ids, one 16-byte load a
+// lane, so that the probe search serves four elements; a group's last ids may
+// lie beyond its list and are masked off.  Workgroups go through the units
+// w, w + gridDim.x, ... and clear the bits they set, so a unit's set costs its
+// d_u ids and not n bits.  The grid is a few times what is resident, so that
+// workgroups share the units evenly.  At n = 262,144 (R-MAT, 8.4M slots) the
+// hub and small block units took 1.65 + 0.29 ms through the HBM bitmaps and
+// the LDS tables, with 0.23 ms for setting and clearing the bitmaps; here 0.86
+// ms.  The limit of ids: at 2^19 (72 KB of LDS, two workgroups a CU) the whole
+// path takes 2.74 against 4.97 ms, at 2^20 (136 KB, one) 11.8 against 12.9 ms
+// and with many small sources more.
+struct LdsBitUnit {
+  uint32_t P[kChunk];   // exclusive prefix of the probes' groups; T beyond the probes
+  uint32_t cb[kChunk];  // first slot of each probe less four times its prefix
+  uint32_t ce[kChunk];  // end of each probe's list
+  int32_t ctr[kChunk];  // hits per probe
+  uint32_t wsum[kWaves];
+  uint32_t pad[8 - kWaves % 8];
+};
+static_assert(sizeof(LdsBitUnit) % 16 == 0, "the bitmap follows aligned");
+
+// Adds each lane's c to ctr[k]; k is nondecreasing over the lanes, so the
+// lanes of one probe are neighbors: an inclusive sum over the wave, and the
+// last lane of each run adds the difference to the sum before the run.
+__device__ __forceinline__ void add_runs(int32_t *ctr, int k, uint32_t c, int lane) {
+  uint32_t x = c;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  const bool head = lane == 0 || k != __shfl_up(k, 1, 64);
+  const unsigned long long heads = __ballot(head);
+  const int start = 63 - __builtin_clzll(heads & ((2ull << lane) - 1));
+  const uint32_t before = __shfl(x, start > 0 ? start - 1 : 0);
+  const bool last = lane == 63 || ((heads >> (lane + 1)) & 1ull);
+  const uint32_t run = x - (start > 0 ? before : 0);
+  if (last && run) __hip_atomic_fetch_add((lds_i32 *)&ctr[k], static_cast<int>(run), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <int U>
+__global__ __launch_bounds__(kWG, 8) void k_bmp_lds(const uint32_t *__restrict__ off, const int32_t *__restrict__ adj,
+                                                    const uint32_t *__restrict__ rev, uint32_t n,
+                                                    const FwdUnit *__restrict__ units, uint32_t n_units,
+                                                    uint32_t words, int32_t *cnt, int plus, unsigned long long *sum) {
+  extern __shared__ __align__(16) unsigned char bmp_lds[];
+  LdsBitUnit &L = *reinterpret_cast<LdsBitUnit *>(bmp_lds);
+  uint32_t *const bits = reinterpret_cast<uint32_t *>(bmp_lds + sizeof(LdsBitUnit));
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned long long total = 0;
+  for (uint32_t i = 4 * tid; i < words; i += 4 * kWG) *reinterpret_cast<uint4 *>(bits + i) = make_uint4(0, 0, 0, 0);
+  __syncthreads();
+  for (uint32_t t = blockIdx.x; t < n_units; t += gridDim.x) {
+    const FwdUnit un = units[t];
+    const uint32_t su = off[un.b], eu = off[un.b + 1];
+    const uint32_t nup = un.j1 - un.j0;
+    uint32_t cb = 0, ce = 0;
+    if (static_cast<uint32_t>(tid) < nup) probe_of(off, adj, n, un.j0 + tid, cb, ce);
+    for (uint32_t i = su + tid; i < eu; i += kWG) {
+      const uint32_t a = static_cast<uint32_t>(adj[i]);
+      if (a < n) lds_or(&bits[a >> 5], 0x80000000u >> (a & 31));
+    }
+    const uint32_t len = (ce - cb + 3) >> 2;
+    const uint32_t excl = wave_excl_scan(len, lane);
+    if (lane == 63) L.wsum[wave] = excl + len;
+    L.ctr[tid] = 0;
+    __syncthreads();
+    uint32_t before = 0, T = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+      const uint32_t ws = L.wsum[w];
+      before += w < wave ? ws : 0;
+      T += ws;
+    }
+    T = __builtin_amdgcn_readfirstlane(T);
+    L.P[tid] = static_cast<uint32_t>(tid) < nup ? before + excl : T;
+    L.cb[tid] = cb - 4 * (before + excl);
+    L.ce[tid] = ce;
+    __syncthreads();
+    constexpr uint32_t kStride = kWaves * 64 * U;
+    struct Round {
+      uint4 v[U];
+      uint32_t left[U];
+      int k[U];
+    };
+    auto fetch = [&](uint32_t f0, Round &r) {
+      const uint32_t f1 = accflat::round_last<U>(f0, T);
+      accflat::lds_search<U>(L.P, f0, f1, lane, r.k);
+#pragma unroll
+      for (int q = 0; q < U; q++) {
+        const uint32_t e = f0 + 64 * q + lane;
+        const uint32_t at = L.cb[r.k[q]] + 4 * min(e, f1);
+        r.left[q] = e < T ? L.ce[r.k[q]] - at : 0;  // ids of the list from here on
+        __builtin_memcpy(&r.v[q], adj + at, 16);    // the array ends with room for the last group
+      }
+    };
+    auto decide = [&](const Round &r) {
+#pragma unroll
+      for (int q = 0; q < U; q++) {
+        const uint32_t a[4] = {r.v[q].x, r.v[q].y, r.v[q].z, r.v[q].w};
+        uint32_t x[4], h = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          x[i] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const unsigned char *>(bits) +
+                                                     ((a[i] >> 3) & 0x1ffffffcu));
+#pragma unroll
+        for (int i = 0; i < 4; i++) h = __builtin_amdgcn_alignbit(h, x[i] << (a[i] & 31), 31);
+        // element i is bit 3 - i
+        const uint32_t left = min(r.left[q], 4u);
+        add_runs(L.ctr, r.k[q], __popc(h >> (4 - left)), lane);
+      }
+    };
+    uint32_t e0 = static_cast<uint32_t>(wave) * 64 * U;
+    if (e0 < T) {
+      // two rounds per turn, one loaded while the other is decided (wave-uniform)
+      Round r0, r1;
+      fetch(e0, r0);
+      for (;;) {
+        const uint32_t e1 = e0 + kStride;
+        if (e1 < T) fetch(e1, r1);
+        decide(r0);
+        if (e1 >= T) break;
+        e0 = e1 + kStride;
+        if (e0 < T) fetch(e0, r0);
+        decide(r1);
+        if (e0 >= T) break;
+      }
+    }
+    __syncthreads();
+    if (static_cast<uint32_t>(tid) < nup) {
+      const int c = L.ctr[tid];
+      total += static_cast<unsigned long long>(c);
+      cnt[un.j0 + tid] = c + plus;
+      const uint32_t p = rev[un.j0 + tid];
+      if (p != ~0u) cnt[p] = c + plus;
+    }
+    for (uint32_t i = su + tid; i < eu; i += kWG) {
+      const uint32_t a = static_cast<uint32_t>(adj[i]);
+      if (a < n) bits[a >> 5] = 0;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+  if (lane == 0 && total) atomicAdd(sum, total);
+}
+
 // ---------------------------------------------------------------- MERGE path
 // Windowed units: N(u) in windows of 2^WBITS sorted ids staged in LDS; per
 // window w, probe k's slice of N(v) holds the ids in [N(u)[w W], N(u)[(w+1) W])
@@ -519,6 +675,16 @@ int launch_bitmap(acc_graph *g, int plus) {
                        p.d_units[kEdgeHash14], p.pool_words, p.idx_shift, g->d_cnt, plus, g->d_sum));
   ACC_TRY(launch_units(k_bmp_hash<15, false>, p.n_units[kEdgeHash15], st, g->d_off, g->d_adj, g->d_rev, g->n,
                        p.d_units[kEdgeHash15], p.pool_words, p.idx_shift, g->d_cnt, plus, g->d_sum));
+  if (hubs_in_lds(g)) {
+    const uint32_t words = static_cast<uint32_t>((p.pool_words + 3) & ~3ull);
+    const uint32_t k = p.n_units[kEdgeHub];
+    if (!k) return ACC_OK;
+    const uint32_t grid = std::min<uint32_t>(k, 16 * std::max(1, g->ctx->num_cus));
+    hipLaunchKernelGGL(k_bmp_lds<kU / 2>, dim3(grid), dim3(kWG), sizeof(LdsBitUnit) + 4 * words, st,
+                       g->d_off, g->d_adj, g->d_rev, g->n, p.d_units[kEdgeHub], k, words, g->d_cnt, plus, g->d_sum);
+    ACC_HIP_TRY(hipGetLastError());
+    return ACC_OK;
+  }
   // hub batches: set the batch's bitmaps, probe its units, clear the bitmaps
   for (size_t k = 0; k + 1 < p.hub_batch.size(); k++) {
     const uint32_t h0 = p.hub_batch[k], h1 = p.hub_batch[k + 1];

@@ -62,9 +62,11 @@ __global__ __launch_bounds__(256) void k_rl_inverse(const uint32_t *__restrict__
 
 // Every non-empty vertex o marks its first slot with o (heads is zeroed
 // first); an inclusive max-scan then gives the source of every slot.  Needs
-// only monotone offsets ending at m.
+// only monotone offsets ending at m.  The adjacency array's kAdjPad ids past
+// its end are set to 0: the last list's 16-byte loads may reach into them.
 __global__ __launch_bounds__(256) void k_rl_heads(const uint32_t *__restrict__ off, uint32_t n,
-                                                  uint32_t *__restrict__ heads) {
+                                                  uint32_t *__restrict__ heads, int32_t *__restrict__ pad) {
+  if (blockIdx.x == 0 && threadIdx.x < kAdjPad) pad[threadIdx.x] = 0;
   for (uint32_t o = blockIdx.x * 256u + threadIdx.x; o < n; o += gridDim.x * 256u) {
     const uint32_t b = off[o];
     if (off[o + 1] > b) heads[b] = o;
@@ -162,7 +164,8 @@ int slot_sources(acc_graph *g) {
   if (e == hipSuccess) e = g->ctx->pool.alloc(&temp, t_bytes ? t_bytes : 1);
   if (e == hipSuccess) e = hipMemsetAsync(heads, 0, sizeof(uint32_t) * m, st);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_rl_heads, dim3(rl_grid(g->n, g->ctx->num_cus)), dim3(256), 0, st, g->d_off, g->n, heads);
+    hipLaunchKernelGGL(k_rl_heads, dim3(rl_grid(g->n, g->ctx->num_cus)), dim3(256), 0, st, g->d_off, g->n, heads,
+                       g->d_adj + m);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipcub::DeviceScan::InclusiveScan(temp, t_bytes, heads, src, hipcub::Max(), m, st);

@@ -116,7 +116,8 @@ int acc_cn_timings(acc_graph *g, float *ms, int cap, char *names, int names_cap)
                                   looping over the tasks (persistent; default 256) */
 #define ACC_PARAM_BMP_HASH_MAX 7 /* bitmap path: sources with d_u at most this (0..16384, default 256) keep
                                     N(u) in an LDS hash table, larger ones in an HBM bitmap; both behind an
-                                    LDS index of N(u) */
+                                    LDS index of N(u).  Up to 2^19 vertices the bitmap lies in LDS, for
+                                    workgroup units with d_u <= 256 too. */
 #define ACC_PARAM_BMP_BATCH 8  /* bitmap path: hub bitmaps built, probed and cleared per batch (1..16384;
                                   the pool of one batch holds at most 8 GiB) */
 int acc_graph_set_param(acc_graph *g, int param, int64_t value);
