@@ -28,12 +28,12 @@
 // atomics.
 //
 // Measured at R-MAT scale 22 (4.2M vertices, 128M slots, 94% of 7.2e9 probe
-// elements at dense sources): counting 4.5 ms + 1.1 ms for the other sources
-// and 1.1 ms for the sums, where the other form took 17.1 ms for all; the
+// elements at dense sources): counting 4.4 ms + 1.1 ms for the other sources
+// and 0.8 ms for the sums, where the other form took 17.1 ms for all; the
 // copy to the upper slots 1.25 ms against 2.2 ms for adding both; the whole
-// pass 20.0 to 8.0 ms.  The triangle-only pass, 6.1 to 3.6 ms, is bound by the
-// lists' traffic (16-bit ids halve it), the per-slot counting by VALU (69% busy)
-// and LDS (55%).
+// pass 20.0 to 7.7 ms.  The triangle-only pass, 6.1 to 3.3 ms, is bound by the
+// lists' traffic (16-bit ids halve it; 18 GB fetched), the per-slot counting by VALU (74%
+// busy) and LDS (58%); its hit bytes and (b, a) counters cost 0.8 ms each.
 
 #include <hip/hip_runtime.h>
 
@@ -52,7 +52,7 @@ using accfwd::kWaves;
 
 constexpr uint32_t kCtrCap = 2048;    // (b, a) counters in LDS; positions beyond update the slot itself
 constexpr uint32_t kRowSmall = 32;    // matrices of at most this many rows: two vertices a wave,
-constexpr uint32_t kRowMid = 256;     // at most this many: one wave each, more: one workgroup each
+constexpr uint32_t kRowMid = 1024;    // at most this many: one wave each, more: one workgroup each
 constexpr int kDenseU = 2;             // rows of 64 groups per round: 16-byte loads in flight per lane
 constexpr uint32_t kNoRows = ~0u;     // hit base of a vertex whose matrix is not kept
 
@@ -106,12 +106,16 @@ __device__ __forceinline__ void lds_or(uint32_t *p, uint32_t v) {
 // ---------------------------------------------------------------- tables
 // Per vertex v (of a graph with first vertex base and limit dense sources): the
 // number of lower neighbors below base + limit (rows) and the 8-id groups of
-// its low list.
+// its low list's place: whole 128-byte lines of 8 groups for a list of more than
+// 4 (wide), which starts on a line; 4, 2 or 1 groups after all of those for a
+// shorter one.  A probe then reads the lines its elements fill and not one
+// more (R-MAT scale 22, triangle-only pass: 3.6 to 3.3 ms).
 __global__ __launch_bounds__(256) void k_dense_count(const uint32_t *__restrict__ off, const uint32_t *__restrict__ hs,
                                                      const int32_t *__restrict__ adj, uint32_t n,
                                                      const uint32_t *__restrict__ gvoff,
                                                      const uint32_t *__restrict__ glimit, uint32_t graphs,
-                                                     uint32_t *__restrict__ rows, uint32_t *__restrict__ groups) {
+                                                     uint32_t *__restrict__ rows, uint32_t *__restrict__ wide,
+                                                     uint32_t *__restrict__ narrow) {
   for (uint32_t v = blockIdx.x * 256u + threadIdx.x; v <= n; v += gridDim.x * 256u) {
     uint32_t r = 0;
     if (v < n) {
@@ -130,8 +134,16 @@ __global__ __launch_bounds__(256) void k_dense_count(const uint32_t *__restrict_
       r = a - s;
       rows[v] = r;
     }
-    groups[v] = (r + 7) >> 3;
+    const uint32_t G = (r + 7) >> 3;
+    wide[v] = G > 4 ? (G + 7) & ~7u : 0;
+    narrow[v] = G > 4 ? 0 : G == 3 ? 4 : G;
   }
+}
+
+// The first group of v's low list, from the prefixes of the wide and narrow places.
+__device__ __forceinline__ uint32_t low_group(const uint32_t *__restrict__ wide0, const uint32_t *__restrict__ narrow0,
+                                              uint32_t v, uint32_t n, uint32_t rows) {
+  return rows > 32 ? wide0[v] : wide0[n] + narrow0[v];
 }
 
 // What the host needs of the tables: the matrices' total bytes, the lengths
@@ -152,9 +164,10 @@ __device__ __forceinline__ int list_of(uint32_t rows, uint32_t cap) {
 // Bytes of every vertex's matrix: 0 where it has none (under two rows) or is
 // not kept (more than cap rows); and their sum and the lists' lengths, with
 // one atomic each per workgroup of a small grid, since atomics on one address
-// queue.  group0 is the finished prefix of the low groups.
+// queue.  wide0 and narrow0 are the finished prefixes of the low groups.
 __global__ __launch_bounds__(256) void k_dense_bytes(const uint32_t *__restrict__ rows,
-                                                     const uint32_t *__restrict__ group0, uint32_t n, uint32_t cap,
+                                                     const uint32_t *__restrict__ wide0,
+                                                     const uint32_t *__restrict__ narrow0, uint32_t n, uint32_t cap,
                                                      uint32_t *__restrict__ bytes, DenseSizes *__restrict__ sizes) {
   __shared__ unsigned long long part[4];
   __shared__ uint32_t len[2];
@@ -175,7 +188,7 @@ __global__ __launch_bounds__(256) void k_dense_bytes(const uint32_t *__restrict_
   if (threadIdx.x == 0) {
     sum = part[0] + part[1] + part[2] + part[3];
     if (sum) atomicAdd(&sizes->bytes, sum);
-    if (blockIdx.x == 0) sizes->groups = group0[n];
+    if (blockIdx.x == 0) sizes->groups = wide0[n] + narrow0[n];
   }
   if (threadIdx.x < 2 && len[threadIdx.x]) atomicAdd(&sizes->lists[threadIdx.x], len[threadIdx.x]);
 }
@@ -212,7 +225,8 @@ __global__ __launch_bounds__(256) void k_dense_fill(const uint32_t *__restrict__
                                                     uint32_t n, const uint32_t *__restrict__ gvoff,
                                                     const uint32_t *__restrict__ glimit, uint32_t graphs,
                                                     const uint32_t *__restrict__ rows,
-                                                    const uint32_t *__restrict__ group0,
+                                                    const uint32_t *__restrict__ wide0,
+                                                    const uint32_t *__restrict__ narrow0,
                                                     const uint32_t *__restrict__ byte0, uint32_t cap,
                                                     uint4 *__restrict__ vmeta, uint4 *__restrict__ low) {
   const int lane = threadIdx.x & 63;
@@ -231,7 +245,7 @@ __global__ __launch_bounds__(256) void k_dense_fill(const uint32_t *__restrict__
       limit = glimit[lo];
       o = off[v];
       r = rows[v];
-      g0 = group0[v];
+      g0 = low_group(wide0, narrow0, v, n, r);
       vmeta[v] = make_uint4(o, g0, r > cap ? kNoRows : byte0[v], r);
     }
     const uint32_t G = wave_excl_scan((r + 7) >> 3, lane);
@@ -243,15 +257,16 @@ __global__ __launch_bounds__(256) void k_dense_fill(const uint32_t *__restrict__
       const uint32_t kbase = __shfl(base, k), klimit = __shfl(limit, k);
       if (e < total) {
         const uint32_t i0 = 8 * (e - kG);
+        int32_t in[8];  // the array ends with room for the last list's group
+        __builtin_memcpy(in, adj + ko + i0, sizeof(in));
         uint32_t w[4];
 #pragma unroll
         for (int h = 0; h < 4; h++) {
           uint32_t id[2];
 #pragma unroll
           for (int x = 0; x < 2; x++) {
-            const uint32_t i = i0 + 2 * h + x;
-            const uint32_t a = i < kr ? static_cast<uint32_t>(adj[ko + i]) - kbase : klimit;
-            id[x] = a < klimit ? a : klimit;  // an id outside (unsorted trusted input) reads as padding
+            const uint32_t a = static_cast<uint32_t>(in[2 * h + x]) - kbase;
+            id[x] = i0 + 2 * h + x < kr && a < klimit ? a : klimit;  // an id outside reads as padding
           }
           w[h] = id[0] | (id[1] << 16);
         }
@@ -379,6 +394,7 @@ __global__ __launch_bounds__(kWG, 8) void k_dense(const uint4 *__restrict__ vmet
           r.v[q] = low[S.cb[r.k[q]] + min(e, f1)];  // past T: the round's last group
         }
       };
+      const bool wide = __builtin_amdgcn_readfirstlane(nl) > ctr_cap;  // positions beyond the LDS counters
       const bool unit_direct = kSlots && __builtin_amdgcn_readfirstlane(S.direct) != 0;
       auto decide = [&](uint32_t f0, const Round &r) {
 #pragma unroll
@@ -409,7 +425,7 @@ __global__ __launch_bounds__(kWG, 8) void k_dense(const uint4 *__restrict__ vmet
               const uint32_t upto =
                   *reinterpret_cast<const uint16_t *>(reinterpret_cast<const unsigned char *>(S.upto) + (w[i] >> 1));
               const uint32_t pos = upto - __popc(x[i]);
-              if (pos < ctr_cap)
+              if (!wide || pos < ctr_cap)
                 lds_add(&S.ctr[pos], 1);
               else
                 atomicAdd(&cnt[mb.x + pos], 1);
@@ -479,29 +495,58 @@ __device__ __forceinline__ uint32_t row_word(const uint8_t *__restrict__ H, uint
   return left >= 4 ? x : x & ((1u << (8 * left)) - 1);
 }
 
-// Sums of the 32 columns of a word, kept as four bytes in each of eight
-// words: byte j of a[k] counts column 8 j + 7 - k (element i of a group is bit
-// 7 - i of its byte), for up to 255 rows.
+// Sums of the 32 columns of a word.  Four rows at a time go through
+// carry-save adders into a word of ones, one of twos and a carry of fours; the
+// carries are counted in the four bytes of eight words, byte j of a[k] for column
+// 8 j + 7 - k (element i of a group is bit 7 - i of its byte): 37 instructions
+// for four rows, where counting every row in the bytes takes 96.
 struct ColumnSums {
+  uint32_t ones = 0, twos = 0;
   uint32_t a[8] = {};
-  __device__ __forceinline__ void add(uint32_t x) {
+  static __device__ __forceinline__ uint32_t carry(uint32_t x, uint32_t y, uint32_t z) { return (x & y) | (z & (x ^ y)); }
+  __device__ __forceinline__ void add(const uint32_t (&x)[4]) {
+    const uint32_t t0 = carry(x[0], x[1], ones);
+    ones ^= x[0] ^ x[1];
+    const uint32_t t1 = carry(x[2], x[3], ones);
+    ones ^= x[2] ^ x[3];
+    const uint32_t f = carry(t0, t1, twos);
+    twos ^= t0 ^ t1;
 #pragma unroll
-    for (int k = 0; k < 8; k++) a[k] += (x >> k) & 0x01010101u;
+    for (int k = 0; k < 8; k++) a[k] += (f >> k) & 0x01010101u;
+  }
+  // Adds the sums over the lanes of a column (lane mod 2^log) to to[0 .. 31]
+  // and starts again.  At most 255 rows in all since the last time, so that the
+  // bytes hold the sums; every lane calls it.  (Left to LDS atomics, the lanes of a
+  // column queue on one address: the kernel took 1.35 ms.)
+  __device__ __forceinline__ void flush(uint32_t *to, int log, bool in, int lane) {
+    uint32_t v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = 4 * a[k] + 2 * ((twos >> k) & 0x01010101u) + ((ones >> k) & 0x01010101u);
+    for (int o = 1 << log; o < 64; o <<= 1)
+#pragma unroll
+      for (int k = 0; k < 8; k++) v[k] += __shfl_xor(v[k], o, 64);
+    if (in && lane < (1 << log)) {
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) lds_add(&to[8 * j + 7 - k], (v[k] >> (8 * j)) & 255u);
+    }
+    *this = ColumnSums{};
   }
 };
 
-// One large or medium matrix of d rows: 2^log lanes per row, one word each
-// (64 words, 2048 columns, per tile), 64 >> log rows a step; `waves` waves
-// take turns at the steps.  Row sums go to sums[t]; column sums are flushed
-// to sums[] by LDS atomics (kBlock) or, for one wave and at most 255 rows,
-// added over the lanes first and then stored by the lanes of the first row.
-template <bool kBlock>
+// One large or medium matrix of d rows in tiles of kTileWords words (256
+// columns), from the tile's first column down, so that little of the triangle
+// above the diagonal is read as nothing: 2^log lanes per row, one word each,
+// 64 >> log rows a step, kTurns waves taking turns at the steps.  Row and column sums
+// are added to sums[] in LDS.
+constexpr uint32_t kTileWords = 8;
+template <uint32_t kTurns>
 __device__ __forceinline__ void sum_matrix(const uint8_t *__restrict__ H, uint32_t d, uint32_t *sums, int wave,
                                            int lane) {
-  constexpr uint32_t kTurns = kBlock ? 4 : 1;
   constexpr int kRows = 4;  // rows in flight per lane
-  for (uint32_t col0 = 0; col0 < d; col0 += 2048) {
-    const uint32_t words = min(64u, (d - col0 + 31) / 32);
+  for (uint32_t col0 = 0; col0 < d; col0 += 32 * kTileWords) {
+    const uint32_t words = min(kTileWords, (d - col0 + 31) / 32);
     const int log = words > 1 ? 32 - __builtin_clz(words - 1) : 0;
     const uint32_t rpw = 64u >> log;
     const uint32_t q = lane & ((1u << log) - 1);
@@ -509,18 +554,7 @@ __device__ __forceinline__ void sum_matrix(const uint8_t *__restrict__ H, uint32
     const bool last = q == (1u << log) - 1;
     const uint32_t step = kTurns * rpw;
     ColumnSums c;
-    uint32_t rounds = 0;
-    auto flush = [&]() {
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const uint32_t v = (c.a[k] >> (8 * j)) & 255u;
-          if (v) lds_add(&sums[32 * w + 8 * j + 7 - k], v);
-        }
-      c = ColumnSums{};
-      rounds = 0;
-    };
+    uint32_t added = 0;
     // wave-uniform loop; every lane reaches the reductions
     for (uint32_t t0 = col0 + wave * rpw; t0 < d; t0 += kRows * step) {
       uint32_t x[kRows];
@@ -529,41 +563,60 @@ __device__ __forceinline__ void sum_matrix(const uint8_t *__restrict__ H, uint32
         const uint32_t t = t0 + step * r + (lane >> log);
         x[r] = t < d ? row_word(H, t, w) : 0;
       }
+      if (added + kRows * rpw > 255) {
+        c.flush(sums + 32 * w, log, 32 * w < d, lane);
+        added = 0;
+      }
 #pragma unroll
       for (int r = 0; r < kRows; r += 2) {
-        // two rows' sums (at most 2048 each) in one word
+        // two rows' sums (at most 256 each) in one word
         const uint32_t rs = group_sum(__popc(x[r]) | (__popc(x[r + 1]) << 16), log);
         const uint32_t t = t0 + step * r + (lane >> log);
         if (last && (rs & 0xffffu)) lds_add(&sums[t], rs & 0xffffu);
         if (last && (rs >> 16)) lds_add(&sums[t + step], rs >> 16);
       }
-#pragma unroll
-      for (int r = 0; r < kRows; r++) c.add(x[r]);
-      if (kBlock && ++rounds == 255 / kRows) flush();
+      c.add(x);
+      added += kRows * rpw;
     }
-    if (kBlock) {
-      flush();
-    } else {
-      for (uint32_t o = 1u << log; o < 64; o <<= 1)
-#pragma unroll
-        for (int k = 0; k < 8; k++) c.a[k] += __shfl_xor(c.a[k], o, 64);
-      if (static_cast<uint32_t>(lane) < (1u << log)) {
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) lds_add(&sums[32 * w + 8 * j + 7 - k], (c.a[k] >> (8 * j)) & 255u);
-      }
-    }
+    c.flush(sums + 32 * w, log, 32 * w < d, lane);
   }
 }
 
+// x of the lane whose number differs in the bits of M (within 32 lanes).
+template <int M>
+__device__ __forceinline__ uint32_t swizzle_xor(uint32_t x) {
+  return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(static_cast<int>(x), (M << 10) | 0x1f));
+}
+
+// The transpose of the 32 x 32 bits held one row per lane by each half of the
+// wave (t = lane mod 32): bit p of lane t becomes bit t of lane p.  Step J
+// exchanges the off-diagonal J x J blocks of every 2J x 2J block.
+template <int J>
+__device__ __forceinline__ uint32_t transpose_step(uint32_t x, uint32_t t) {
+  constexpr uint32_t kLow = J == 16 ? 0x0000ffffu : J == 8 ? 0x00ff00ffu : J == 4 ? 0x0f0f0f0fu : J == 2 ? 0x33333333u : 0x55555555u;
+  const uint32_t y = swizzle_xor<J>(x);
+  const bool hi = t & J;
+  const uint32_t keep = hi ? ~kLow : kLow;
+  const uint32_t moved = __builtin_amdgcn_alignbit(y, y, hi ? J : 32 - J);  // rotated right by J, or left
+  return (x & keep) | (moved & ~keep);
+}
+__device__ __forceinline__ uint32_t transpose32(uint32_t x, uint32_t t) {
+  x = transpose_step<16>(x, t);
+  x = transpose_step<8>(x, t);
+  x = transpose_step<4>(x, t);
+  x = transpose_step<2>(x, t);
+  return transpose_step<1>(x, t);
+}
+
 // Adds the row and column sums of every hit matrix to its vertex's lower
-// slots.  Workgroups [0, n_large) take one large matrix each, the next ones
+// slots: 0.81 ms for 0.93 GB of matrices at R-MAT scale 22 (1.12 ms with one
+// tile of all columns per matrix, four waves to it and every row counted in
+// bytes), VALU and the latency of short matrices.  Workgroups [0, n_large) take one large matrix each, the next ones
 // four medium matrices each (one per wave; sum_matrix).  The others go over
 // all vertices for the small ones, `span` vertices a wave (a power of two up
 // to 64): two vertices at a time, lane t of each half holding row t as one
-// word, so that the row sum is a popcount and a column's sum the popcount of
-// a ballot.
+// word; the row sums are popcounts, and the column sums those of the
+// transposed matrix.
 __global__ __launch_bounds__(256) void k_dense_rows(const uint4 *__restrict__ vmeta, uint32_t n,
                                                     const uint32_t *__restrict__ large, uint32_t n_large,
                                                     const uint32_t *__restrict__ mid_v, uint32_t n_mid,
@@ -575,9 +628,9 @@ __global__ __launch_bounds__(256) void k_dense_rows(const uint4 *__restrict__ vm
   if (blockIdx.x < n_large) {
     const uint4 m = vmeta[large[blockIdx.x]];
     const uint32_t d = __builtin_amdgcn_readfirstlane(m.w);
-    for (uint32_t i = threadIdx.x; i < d; i += 256) sums[i] = 0;
+    for (uint32_t i = threadIdx.x; i < ((d + 31) & ~31u); i += 256) sums[i] = 0;
     __syncthreads();
-    sum_matrix<true>(hits + m.z, d, sums, wave, lane);
+    sum_matrix<4>(hits + m.z, d, sums, wave, lane);
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < d; i += 256) {
       const uint32_t v = sums[i];
@@ -592,9 +645,9 @@ __global__ __launch_bounds__(256) void k_dense_rows(const uint4 *__restrict__ vm
     const uint4 m = vmeta[mid_v[i]];
     const uint32_t d = __builtin_amdgcn_readfirstlane(m.w);
     uint32_t *const own = sums + wave * kRowMid;
-    for (uint32_t s = lane; s < kRowMid; s += 64) own[s] = 0;
+    for (uint32_t s = lane; s < ((d + 31) & ~31u); s += 64) own[s] = 0;
     wave_lds_sync();
-    sum_matrix<false>(hits + m.z, d, own, 0, lane);
+    sum_matrix<1>(hits + m.z, d, own, 0, lane);
     wave_lds_sync();
     for (uint32_t s = lane; s < d; s += 64) {
       const uint32_t v = own[s];
@@ -620,13 +673,7 @@ __global__ __launch_bounds__(256) void k_dense_rows(const uint4 *__restrict__ vm
       const uint32_t dk = __shfl(m.w, k);
       const uint32_t d = lane < 32 || two ? dk : 0;
       const uint32_t x = t < d ? row_word(hits + hb, t, 0) : 0;
-      uint32_t c = __popc(x);
-      const uint32_t dm = __builtin_amdgcn_readfirstlane(max(__shfl(m.w, k0), __shfl(m.w, k1)));
-      for (uint32_t s = 0; s + 1 < dm; s++) {  // row t has bits below t: the last column is empty
-        const unsigned long long b = __ballot((x >> (s ^ 7)) & 1u);
-        const uint32_t n0 = __popc(static_cast<uint32_t>(b)), n1 = __popc(static_cast<uint32_t>(b >> 32));
-        if (t == s) c += lane < 32 ? n0 : n1;
-      }
+      const uint32_t c = __popc(x) + swizzle_xor<7>(__popc(transpose32(x, t)));
       if (t < d && c) cnt[o + t] += static_cast<int>(c);
     }
   }
@@ -663,19 +710,20 @@ int build_tables(acc_graph *g) {
   hipStream_t st = g->ctx->stream;
   const int cus = g->ctx->num_cus;
   const size_t n1 = static_cast<size_t>(n) + 1;
-  // scratch: the sizes, rows, groups and their prefix, bytes and their
-  // prefix, the graphs' first vertices and limits
+  // scratch: the sizes, rows, wide and narrow places and their prefixes, bytes
+  // and their prefix, the graphs' first vertices and limits
   size_t t_scan = 0;
   uint32_t *w = nullptr;
   ACC_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, t_scan, w, w, static_cast<int>(n1), st));
-  const size_t words = 8 + 4 * n1 + 2 * static_cast<size_t>(graphs);
+  const size_t words = 8 + 6 * n1 + 2 * static_cast<size_t>(graphs);
   const size_t scan_at = (sizeof(uint32_t) * words + 255) / 256 * 256;
   static_assert(sizeof(DenseSizes) <= 8 * sizeof(uint32_t), "the sizes lie before the rows");
   if (g->ctx->pool.alloc(reinterpret_cast<void **>(&w), scan_at + t_scan + 16) != hipSuccess)
     return acc_set_error(ACC_ENOMEM, "hipMalloc of the dense tables' scratch failed");
   auto *const sizes = reinterpret_cast<DenseSizes *>(w);
   uint32_t *const rows = w + 8;
-  uint32_t *const len = rows + n1, *const group0 = len + n1, *const byte0 = group0 + n1;
+  uint32_t *const wide = rows + n1, *const narrow = wide + n1, *const wide0 = narrow + n1, *const narrow0 = wide0 + n1;
+  uint32_t *const byte0 = narrow0 + n1, *const len = wide;  // the places are done with once summed
   uint32_t *const gvoff = byte0 + n1, *const glimit = gvoff + graphs;
   void *const temp = reinterpret_cast<char *>(w) + scan_at;
   auto fail = [&](int rc) {
@@ -692,10 +740,11 @@ int build_tables(acc_graph *g) {
     e = hipMemcpyAsync(glimit, p.limit.data(), sizeof(uint32_t) * graphs, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_dense_count, dim3(grid_for(n1, cus, 8)), dim3(256), 0, st, g->d_off, g->d_hs, g->d_adj, n,
-                       gvoff, glimit, graphs, rows, len);
+                       gvoff, glimit, graphs, rows, wide, narrow);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(temp, t_scan, len, group0, static_cast<int>(n1), st);
+  if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(temp, t_scan, wide, wide0, static_cast<int>(n1), st);
+  if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(temp, t_scan, narrow, narrow0, static_cast<int>(n1), st);
   // the largest cap whose matrices stay within 32-bit offsets and 16 bytes per slot
   const uint64_t most = std::min<uint64_t>(0xe0000000ull, 16 * g->m + (1u << 20));
   DenseSizes h{};
@@ -704,7 +753,7 @@ int build_tables(acc_graph *g) {
     p.hit_cap /= 2;
     if (e == hipSuccess) e = hipMemsetAsync(sizes, 0, sizeof(DenseSizes), st);
     if (e == hipSuccess) {
-      hipLaunchKernelGGL(k_dense_bytes, dim3(grid_for(n1, cus, 1)), dim3(256), 0, st, rows, group0, n, p.hit_cap, len,
+      hipLaunchKernelGGL(k_dense_bytes, dim3(grid_for(n1, cus, 1)), dim3(256), 0, st, rows, wide0, narrow0, n, p.hit_cap, len,
                          sizes);
       e = hipGetLastError();
     }
@@ -727,7 +776,7 @@ int build_tables(acc_graph *g) {
   e = hipcub::DeviceScan::ExclusiveSum(temp, t_scan, len, byte0, static_cast<int>(n1), st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_dense_fill, dim3(grid_for(static_cast<uint64_t>(n) * 4, cus, 8)), dim3(256), 0, st, g->d_off,
-                       g->d_adj, n, gvoff, glimit, graphs, rows, group0, byte0, p.hit_cap, p.d_vmeta, p.d_low);
+                       g->d_adj, n, gvoff, glimit, graphs, rows, wide0, narrow0, byte0, p.hit_cap, p.d_vmeta, p.d_low);
     e = hipGetLastError();
   }
   if (e == hipSuccess && p.n_large + p.n_mid) {
