@@ -116,6 +116,28 @@ __device__ __forceinline__ void add_row_hits(int32_t *ctr, int k, bool hit, int 
   }
 }
 
+// Adds each lane's c to ctr[k]; k is nondecreasing over the lanes, so the
+// lanes of one probe are neighbors: an inclusive sum over the wave, and the
+// last lane of each run adds the difference to the sum before the run.
+__device__ __forceinline__ void add_runs(int32_t *ctr, int k, uint32_t c, int lane) {
+  uint32_t x = c;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  const int left = __shfl_up(k, 1, 64);
+  const unsigned long long heads = __ballot(lane == 0 || k != left);
+  const int start = 63 - __builtin_clzll(heads & ((2ull << lane) - 1));
+  const uint32_t before = __shfl(x, start > 0 ? start - 1 : 0);
+  const bool last = lane == 63 || ((heads >> (lane + 1)) & 1ull);
+  const uint32_t run = x - (start > 0 ? before : 0);
+  typedef __attribute__((address_space(3))) int32_t lds_i32;
+  if (last && run) __hip_atomic_fetch_add((lds_i32 *)&ctr[k], static_cast<int>(run), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // The round's last element below `end` (end > e0).
 template <int U>
 __device__ __forceinline__ uint32_t round_last(uint32_t e0, uint32_t end) {

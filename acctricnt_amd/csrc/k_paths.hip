@@ -468,27 +468,6 @@ struct LdsBitUnit {
 };
 static_assert(sizeof(LdsBitUnit) % 16 == 0, "the bitmap follows aligned");
 
-// Adds each lane's c to ctr[k]; k is nondecreasing over the lanes, so the
-// lanes of one probe are neighbors: an inclusive sum over the wave, and the
-// last lane of each run adds the difference to the sum before the run.
-__device__ __forceinline__ void add_runs(int32_t *ctr, int k, uint32_t c, int lane) {
-  uint32_t x = c;
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
-  const bool head = lane == 0 || k != __shfl_up(k, 1, 64);
-  const unsigned long long heads = __ballot(head);
-  const int start = 63 - __builtin_clzll(heads & ((2ull << lane) - 1));
-  const uint32_t before = __shfl(x, start > 0 ? start - 1 : 0);
-  const bool last = lane == 63 || ((heads >> (lane + 1)) & 1ull);
-  const uint32_t run = x - (start > 0 ? before : 0);
-  if (last && run) __hip_atomic_fetch_add((lds_i32 *)&ctr[k], static_cast<int>(run), __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 template <int U>
 __global__ __launch_bounds__(kWG, 8) void k_bmp_lds(const uint32_t *__restrict__ off, const int32_t *__restrict__ adj,
                                                     const uint32_t *__restrict__ rev, uint32_t n,
@@ -559,7 +538,7 @@ __global__ __launch_bounds__(kWG, 8) void k_bmp_lds(const uint32_t *__restrict__
         for (int i = 0; i < 4; i++) h = __builtin_amdgcn_alignbit(h, x[i] << (a[i] & 31), 31);
         // element i is bit 3 - i
         const uint32_t left = min(r.left[q], 4u);
-        add_runs(L.ctr, r.k[q], __popc(h >> (4 - left)), lane);
+        accflat::add_runs(L.ctr, r.k[q], __popc(h >> (4 - left)), lane);
       }
     };
     uint32_t e0 = static_cast<uint32_t>(wave) * 64 * U;
