@@ -420,10 +420,11 @@ int load_vertex_meta(acc_graph *g, const uint32_t *host_off) {
   const uint32_t n = g->n;
   ACC_TRY(dev_alloc(g, &g->d_hs, static_cast<uint64_t>(n) + 1));
   int32_t *lo = nullptr;
-  if (g->ctx->pool.alloc(reinterpret_cast<void **>(&lo), sizeof(int32_t) * (static_cast<size_t>(n) + 2)) != hipSuccess)
+  std::vector<uint32_t> h_max(2 * static_cast<size_t>(accfwd::vertex_meta_blocks(g)));
+  if (g->ctx->pool.alloc(reinterpret_cast<void **>(&lo), sizeof(int32_t) * (static_cast<size_t>(n) + h_max.size())) !=
+      hipSuccess)
     return acc_set_error(ACC_ENOMEM, "hipMalloc of the vertex metadata failed");
   uint32_t *d_max = reinterpret_cast<uint32_t *>(lo + n);
-  uint32_t h_max[2] = {0, 0};
   g->h_off.resize(static_cast<size_t>(n) + 1);
   g->h_hs.resize(n);
   g->h_lo.resize(n);
@@ -437,12 +438,15 @@ int load_vertex_meta(acc_graph *g, const uint32_t *host_off) {
   }
   if (!rc) rc = staged_copy(g->ctx, g->h_hs.data(), g->d_hs, sizeof(uint32_t) * n, false);
   if (!rc) rc = staged_copy(g->ctx, g->h_lo.data(), lo, sizeof(int32_t) * n, false);
-  if (!rc) rc = staged_copy(g->ctx, h_max, d_max, sizeof(h_max), false);
+  if (!rc) rc = staged_copy(g->ctx, h_max.data(), d_max, sizeof(uint32_t) * h_max.size(), false);
   (void)hipStreamSynchronize(st);
   g->ctx->pool.free(lo);
   if (rc) return rc;
-  g->max_low = h_max[0];
-  g->max_deg = h_max[1];
+  g->max_low = g->max_deg = 0;
+  for (size_t i = 0; i < h_max.size(); i += 2) {
+    g->max_low = std::max(g->max_low, h_max[i]);
+    g->max_deg = std::max(g->max_deg, h_max[i + 1]);
+  }
   return ACC_OK;
 }
 
