@@ -66,8 +66,31 @@ class DevicePool {
   size_t idle_bytes_ = 0;
 };
 
+// Words of pinned host memory that kernels write results to: a total is there
+// once the stream is synchronized, without a copy.  A call takes a word for as
+// long as it waits; with none left (or none to be had) it copies instead.  Safe from
+// several threads.
+struct HostWord {
+  volatile unsigned long long *host = nullptr;
+  unsigned long long *dev = nullptr;
+};
+class HostWords {
+ public:
+  bool init();
+  bool take(HostWord *w);
+  void give(const HostWord &w);
+  ~HostWords();
+
+ private:
+  static constexpr uint32_t kWords = 64;
+  std::mutex mu_;
+  unsigned long long *base_ = nullptr;
+  std::vector<HostWord> idle_;
+};
+
 struct acc_ctx {
   DevicePool pool;
+  HostWords words;
   int device = 0;
   hipStream_t stream = nullptr;
   int num_cus = 0;
@@ -151,6 +174,7 @@ struct acc_graph {
   unsigned long long *d_sum = nullptr;  // [0]: sum over upper slots of the raw counts (= 3T); [1]: T alone
   int32_t *d_flags = nullptr;           // validation flags
   unsigned long long *d_tri_parts = nullptr;  // partial sums of the triangle-only pass
+  bool tri_parts_zero = false;                // the last pass left them zero
   int32_t *d_src = nullptr;             // source vertex of every slot (built for SCAN)
   int32_t *d_old = nullptr;             // caller vertex ids for cluster ids (NULL: identity)
   // similarity index (built for serving): every vertex's slots sorted by a
@@ -344,7 +368,10 @@ int launch_init(acc_graph *g, int fill);
 // d_flags[2..3] (a uint64) the number of upper slots.
 int launch_build_rev(acc_graph *g, bool validate);
 // Triangle total only (forward path, no per-slot counts) into d_sum[1].
-int launch_triangles(acc_graph *g);
+// The total goes to d_sum[1], and to *copy (device-visible host memory) if given.
+int launch_triangles(acc_graph *g, unsigned long long *copy);
+// *to = *from.
+int launch_publish(acc_graph *g, const unsigned long long *from, unsigned long long *to);
 int launch_count(acc_graph *g);
 int launch_count_big(acc_graph *g);
 // Copies the lower slots' counts to the upper ones or adds the two

@@ -459,6 +459,36 @@ int record_event(acc_graph *g, const char *name) {
   return rc;
 }
 
+bool HostWords::init() {
+  std::lock_guard<std::mutex> lk(mu_);
+  void *dev = nullptr;
+  if (hipHostMalloc(reinterpret_cast<void **>(&base_), sizeof(unsigned long long) * kWords,
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    base_ = nullptr;
+    return false;
+  }
+  if (hipHostGetDevicePointer(&dev, base_, 0) != hipSuccess) return false;
+  for (uint32_t i = 0; i < kWords; i++) idle_.push_back({base_ + i, static_cast<unsigned long long *>(dev) + i});
+  return true;
+}
+
+bool HostWords::take(HostWord *w) {
+  std::lock_guard<std::mutex> lk(mu_);
+  if (idle_.empty()) return false;
+  *w = idle_.back();
+  idle_.pop_back();
+  return true;
+}
+
+void HostWords::give(const HostWord &w) {
+  std::lock_guard<std::mutex> lk(mu_);
+  idle_.push_back(w);
+}
+
+HostWords::~HostWords() {
+  if (base_) (void)hipHostFree(base_);
+}
+
 hipError_t DevicePool::alloc(void **p, size_t bytes) {
   *p = nullptr;
   const size_t step = bytes > (size_t(1) << 20) ? size_t(64) << 10 : size_t(4) << 10;
@@ -556,6 +586,7 @@ int acc_ctx_create(int device, acc_ctx **out) {
     delete ctx;
     return rc;
   }
+  if (!ctx->words.init()) (void)hipGetLastError();  // totals are copied then
   *out = ctx;
   return ACC_OK;
 }
@@ -741,10 +772,18 @@ int acc_cn_download(acc_graph *g, int32_t *cnt_host, uint64_t *triangles) {
   if (!g) return acc_set_error(ACC_EINVAL, "null graph");
   if (!g->have_result) return acc_set_error(ACC_EINVAL, "no counts computed yet");
   DeviceGuard guard(g->ctx->device);
+  HostWord w;
+  const bool word = triangles && g->ctx->words.take(&w);
+  // a word that a kernel may still write to (an error below) is not given back
+  if (word) ACC_TRY(accfwd::launch_publish(g, g->d_sum, w.dev));
   if (cnt_host && g->m) ACC_TRY(staged_copy(g->ctx, cnt_host, g->d_cnt, sizeof(int32_t) * g->m, false));
   unsigned long long s = 0;
-  ACC_HIP_TRY(hipMemcpyAsync(&s, g->d_sum, sizeof(s), hipMemcpyDeviceToHost, g->ctx->stream));
+  if (!word) ACC_HIP_TRY(hipMemcpyAsync(&s, g->d_sum, sizeof(s), hipMemcpyDeviceToHost, g->ctx->stream));
   ACC_HIP_TRY(hipStreamSynchronize(g->ctx->stream));
+  if (word) {
+    s = *w.host;
+    g->ctx->words.give(w);
+  }
   if (triangles) *triangles = s / 3;
   return ACC_OK;
 }
@@ -1125,10 +1164,16 @@ int acc_triangle_total(acc_graph *g, int path, uint64_t *triangles) {
   }
   // forward lists without per-slot outputs: every triangle counted once at its middle vertex
   DeviceGuard guard(g->ctx->device);
-  ACC_TRY(accfwd::launch_triangles(g));
+  HostWord w;
+  const bool word = g->ctx->words.take(&w);
+  ACC_TRY(accfwd::launch_triangles(g, word ? w.dev : nullptr));
   unsigned long long t = 0;
-  ACC_HIP_TRY(hipMemcpyAsync(&t, g->d_sum + 1, sizeof(t), hipMemcpyDeviceToHost, g->ctx->stream));
+  if (!word) ACC_HIP_TRY(hipMemcpyAsync(&t, g->d_sum + 1, sizeof(t), hipMemcpyDeviceToHost, g->ctx->stream));
   ACC_HIP_TRY(hipStreamSynchronize(g->ctx->stream));
+  if (word) {  // after an error it may still be written to and is not given back
+    t = *w.host;
+    g->ctx->words.give(w);
+  }
   *triangles = t;
   return ACC_OK;
 }
@@ -1136,7 +1181,7 @@ int acc_triangle_total(acc_graph *g, int path, uint64_t *triangles) {
 int acc_triangle_launch(acc_graph *g) {
   if (!g) return acc_set_error(ACC_EINVAL, "null graph");
   DeviceGuard guard(g->ctx->device);
-  return accfwd::launch_triangles(g);
+  return accfwd::launch_triangles(g, nullptr);
 }
 
 }  // extern "C"

@@ -849,18 +849,24 @@ __global__ __launch_bounds__(kTriParts) void k_tri_zero(unsigned long long *__re
   parts[threadIdx.x * kTriStride] = 0;
 }
 
-__global__ __launch_bounds__(kTriParts) void k_tri_sum(const unsigned long long *__restrict__ parts,
-                                                       unsigned long long *__restrict__ total) {
+// The total of the parts, which are left zero for the next pass.
+__global__ __launch_bounds__(kTriParts) void k_tri_sum(unsigned long long *__restrict__ parts,
+                                                       unsigned long long *__restrict__ total,
+                                                       unsigned long long *__restrict__ copy) {
   __shared__ unsigned long long w[kTriParts / 64];
   const unsigned long long v = wave_sum_u64(parts[threadIdx.x * kTriStride]);
+  parts[threadIdx.x * kTriStride] = 0;
   if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
     unsigned long long t = 0;
     for (int i = 0; i < kTriParts / 64; i++) t += w[i];
     *total = t;
+    if (copy) *copy = t;
   }
 }
+
+__global__ void k_publish(const unsigned long long *__restrict__ from, unsigned long long *__restrict__ to) { *to = *from; }
 
 __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long *__restrict__ p, uint32_t count) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -1087,7 +1093,13 @@ int launch_count(acc_graph *g) { return launch_count_t<true>(g, nullptr); }
 
 int launch_count_big(acc_graph *g) { return launch_big_t<true>(g, nullptr); }
 
-int launch_triangles(acc_graph *g) {
+int launch_publish(acc_graph *g, const unsigned long long *from, unsigned long long *to) {
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, g->ctx->stream, from, to);
+  ACC_HIP_TRY(hipGetLastError());
+  return ACC_OK;
+}
+
+int launch_triangles(acc_graph *g, unsigned long long *copy) {
   ACC_TRY(accdense::ensure(g, false));
   if (!g->d_tri_parts) {
     if (g->ctx->pool.alloc(reinterpret_cast<void **>(&g->d_tri_parts),
@@ -1098,13 +1110,25 @@ int launch_triangles(acc_graph *g) {
     g->device_bytes += sizeof(unsigned long long) * kTriParts * kTriStride;
   }
   hipStream_t st = g->ctx->stream;
-  hipLaunchKernelGGL(k_tri_zero, dim3(1), dim3(kTriParts), 0, st, g->d_tri_parts);
-  ACC_HIP_TRY(hipGetLastError());
+  // Every pass leaves the parts zero (k_tri_sum), so only the first one after
+  // their allocation or after a pass that was not launched whole zeroes them: a
+  // launch less in a call that is little more than its launches.  A stream
+  // recorded by a caller runs nothing yet, so its pass zeroes them itself and
+  // leaves the next one to do so too.
+  hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+  ACC_HIP_TRY(hipStreamIsCapturing(st, &recording));
+  const bool zero = !g->tri_parts_zero || recording != hipStreamCaptureStatusNone;
+  g->tri_parts_zero = false;
+  if (zero) {
+    hipLaunchKernelGGL(k_tri_zero, dim3(1), dim3(kTriParts), 0, st, g->d_tri_parts);
+    ACC_HIP_TRY(hipGetLastError());
+  }
   ACC_TRY(accdense::launch_triangles(g, g->d_tri_parts));
   ACC_TRY(launch_count_t<false>(g, g->d_tri_parts));
   ACC_TRY(launch_big_t<false>(g, g->d_tri_parts));
-  hipLaunchKernelGGL(k_tri_sum, dim3(1), dim3(kTriParts), 0, st, g->d_tri_parts, g->d_sum + 1);
+  hipLaunchKernelGGL(k_tri_sum, dim3(1), dim3(kTriParts), 0, st, g->d_tri_parts, g->d_sum + 1, copy);
   ACC_HIP_TRY(hipGetLastError());
+  g->tri_parts_zero = recording == hipStreamCaptureStatusNone;
   return ACC_OK;
 }
 
