@@ -171,7 +171,7 @@ struct acc_graph {
   int32_t *d_cnt = nullptr;
   uint32_t *d_hs = nullptr;             // first upper slot of every vertex
   uint32_t *d_rev = nullptr;            // reverse slot of every upper slot, ~0 elsewhere (built at upload)
-  unsigned long long *d_sum = nullptr;  // [0]: sum over upper slots of the raw counts (= 3T); [1]: T alone
+  unsigned long long *d_sum = nullptr;  // sum over upper slots of the raw counts (3T) in sum_parts; [1]: T alone
   int32_t *d_flags = nullptr;           // validation flags
   unsigned long long *d_tri_parts = nullptr;  // partial sums of the triangle-only pass
   bool tri_parts_zero = false;                // the last pass left them zero
@@ -355,6 +355,11 @@ namespace accfwd {
 // 128-byte line apart, workgroup w adding into counter w mod kTriParts, so
 // the atomics of many small units do not queue on one address.
 constexpr int kTriParts = 256;
+// A pass's total likewise, in kSumParts counters at sum_parts(g): d_sum[0] takes
+// their sum where no pinned word is to be had, d_sum[1] the triangle-only total.
+constexpr int kSumParts = 64;
+constexpr int kSumStride = 16;
+inline unsigned long long *sum_parts(const acc_graph *g) { return g->d_sum + kSumStride; }
 constexpr int kTriStride = 16;  // unsigned long longs per 128-byte line
 // Whether a pass collects every edge's count in its lower slot, which the
 // combine copies to the upper one.  Otherwise (an upload trusted without
@@ -370,8 +375,8 @@ int launch_build_rev(acc_graph *g, bool validate);
 // Triangle total only (forward path, no per-slot counts) into d_sum[1].
 // The total goes to d_sum[1], and to *copy (device-visible host memory) if given.
 int launch_triangles(acc_graph *g, unsigned long long *copy);
-// *to = *from.
-int launch_publish(acc_graph *g, const unsigned long long *from, unsigned long long *to);
+// *to = the sum of the pass's total counters.
+int launch_publish(acc_graph *g, unsigned long long *to);
 int launch_count(acc_graph *g);
 int launch_count_big(acc_graph *g);
 // Copies the lower slots' counts to the upper ones or adds the two

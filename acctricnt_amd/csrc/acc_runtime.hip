@@ -649,7 +649,7 @@ int acc_graph_upload(acc_ctx *ctx, uint32_t n, uint64_t m, const uint32_t *node_
   if ((rc = dev_alloc(g, &g->d_adj, m + kAdjPad))) return bail(rc);
   if ((rc = dev_alloc(g, &g->d_cnt, m + 4))) return bail(rc);
   if ((rc = dev_alloc(g, &g->d_rev, m + 4))) return bail(rc);
-  if ((rc = dev_alloc(g, &g->d_sum, 2))) return bail(rc);
+  if ((rc = dev_alloc(g, &g->d_sum, accfwd::kSumStride * (1 + accfwd::kSumParts)))) return bail(rc);
   if ((rc = dev_alloc(g, &g->d_flags, 4))) return bail(rc);
   if ((rc = staged_copy(ctx, g->d_off, node_off, sizeof(uint32_t) * (static_cast<size_t>(n) + 1), true)))
     return bail(rc);
@@ -775,10 +775,11 @@ int acc_cn_download(acc_graph *g, int32_t *cnt_host, uint64_t *triangles) {
   HostWord w;
   const bool word = triangles && g->ctx->words.take(&w);
   // a word that a kernel may still write to (an error below) is not given back
-  if (word) ACC_TRY(accfwd::launch_publish(g, g->d_sum, w.dev));
+  if (triangles) ACC_TRY(accfwd::launch_publish(g, word ? w.dev : g->d_sum));
   if (cnt_host && g->m) ACC_TRY(staged_copy(g->ctx, cnt_host, g->d_cnt, sizeof(int32_t) * g->m, false));
   unsigned long long s = 0;
-  if (!word) ACC_HIP_TRY(hipMemcpyAsync(&s, g->d_sum, sizeof(s), hipMemcpyDeviceToHost, g->ctx->stream));
+  if (triangles && !word)
+    ACC_HIP_TRY(hipMemcpyAsync(&s, g->d_sum, sizeof(s), hipMemcpyDeviceToHost, g->ctx->stream));
   ACC_HIP_TRY(hipStreamSynchronize(g->ctx->stream));
   if (word) {
     s = *w.host;

@@ -53,7 +53,7 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
   return v;
 }
 
-// Sets the counts to `fill` and clears the triangle sum and the per-graph totals
+// Sets the counts to `fill` and clears the counters of the total and the per-graph totals
 // of a partitioned graph (parts of them; gtot may be NULL when parts is 0).
 __global__ __launch_bounds__(256) void k_init(int32_t *__restrict__ cnt, uint64_t m, int fill,
                                               unsigned long long *__restrict__ sum,
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void k_init(int32_t *__restrict__ cnt, uint64_
   for (uint64_t i = tid; i < m4; i += stride) reinterpret_cast<int4 *>(cnt)[i] = z;
   for (uint64_t i = m4 * 4 + tid; i < m; i += stride) cnt[i] = fill;
   for (uint64_t k = tid; k < parts; k += stride) gtot[k] = 0;
-  if (tid == 0) *sum = 0;
+  if (tid < accfwd::kSumParts) sum[tid * accfwd::kSumStride] = 0;
 }
 
 // Forward work estimate of every source b: over its upper slots (b, c) the
@@ -841,7 +841,7 @@ __global__ __launch_bounds__(256) void k_combine(int32_t *__restrict__ cnt, cons
   __syncthreads();
   if (threadIdx.x == 0) {
     const unsigned long long t = part[0] + part[1] + part[2] + part[3];
-    if (t) atomicAdd(sum, t);
+    if (t) atomicAdd(accflat::sum_part(sum), t);
   }
 }
 
@@ -866,7 +866,12 @@ __global__ __launch_bounds__(kTriParts) void k_tri_sum(unsigned long long *__res
   }
 }
 
-__global__ void k_publish(const unsigned long long *__restrict__ from, unsigned long long *__restrict__ to) { *to = *from; }
+__global__ __launch_bounds__(64) void k_publish(const unsigned long long *__restrict__ parts,
+                                                unsigned long long *__restrict__ to) {
+  static_assert(accfwd::kSumParts == 64, "one counter per lane");
+  const unsigned long long t = wave_sum_u64(parts[threadIdx.x * accfwd::kSumStride]);
+  if (threadIdx.x == 0) *to = t;
+}
 
 __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long *__restrict__ p, uint32_t count) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -971,7 +976,7 @@ __global__ __launch_bounds__(256) void k_combine_parts(int32_t *__restrict__ cnt
     s0 = e;
     k++;
   }
-  if (threadIdx.x == 0 && all) atomicAdd(sum, all);
+  if (threadIdx.x == 0 && all) atomicAdd(accflat::sum_part(sum), all);
 }
 
 // Flags: 1 id out of range, 2 self-loop, 4 unsorted (duplicates included).
@@ -1009,7 +1014,7 @@ namespace accfwd {
 
 int launch_init(acc_graph *g, int fill) {
   hipLaunchKernelGGL(k_init, dim3(grid_for(g->m / 4 + 1, g->ctx->num_cus)), dim3(256), 0, g->ctx->stream,
-                     g->d_cnt, g->m, fill, g->d_sum, g->num_parts ? g->d_gtot : nullptr, g->num_parts);
+                     g->d_cnt, g->m, fill, sum_parts(g), g->num_parts ? g->d_gtot : nullptr, g->num_parts);
   ACC_HIP_TRY(hipGetLastError());
   return ACC_OK;
 }
@@ -1093,8 +1098,8 @@ int launch_count(acc_graph *g) { return launch_count_t<true>(g, nullptr); }
 
 int launch_count_big(acc_graph *g) { return launch_big_t<true>(g, nullptr); }
 
-int launch_publish(acc_graph *g, const unsigned long long *from, unsigned long long *to) {
-  hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, g->ctx->stream, from, to);
+int launch_publish(acc_graph *g, unsigned long long *to) {
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, g->ctx->stream, sum_parts(g), to);
   ACC_HIP_TRY(hipGetLastError());
   return ACC_OK;
 }
@@ -1138,13 +1143,13 @@ int launch_combine(acc_graph *g, int plus) {
     if (g->m) {
       const uint32_t blocks = static_cast<uint32_t>((g->m + kCombSpan - 1) / kCombSpan);
       hipLaunchKernelGGL((gather ? k_combine_parts<true> : k_combine_parts<false>), dim3(blocks), dim3(256), 0, g->ctx->stream, g->d_cnt, g->d_rev,
-                         static_cast<uint32_t>(g->m), plus, g->d_sum, g->d_gsoff, g->num_parts, g->d_gtot);
+                         static_cast<uint32_t>(g->m), plus, sum_parts(g), g->d_gsoff, g->num_parts, g->d_gtot);
     }
     ACC_HIP_TRY(hipGetLastError());
     return ACC_OK;
   }
   hipLaunchKernelGGL((gather ? k_combine<true> : k_combine<false>), dim3(grid_for(g->m, g->ctx->num_cus)), dim3(256), 0,
-                     g->ctx->stream, g->d_cnt, g->d_rev, g->m, plus, g->d_sum);
+                     g->ctx->stream, g->d_cnt, g->d_rev, g->m, plus, sum_parts(g));
   ACC_HIP_TRY(hipGetLastError());
   return ACC_OK;
 }

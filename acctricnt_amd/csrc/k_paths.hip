@@ -130,7 +130,7 @@ __device__ __forceinline__ void probe_flat(const int32_t *__restrict__ adj, cons
 }
 
 // Writes each probe's count into its upper slot and reverse slot and adds
-// the unit's raw counts to *sum.  Follows a __syncthreads.
+// the unit's raw counts to the total.  Follows a __syncthreads.
 __device__ __forceinline__ void finish_unit(const UnitLds &L, const uint32_t *__restrict__ rev, uint32_t j0,
                                             uint32_t nup, int32_t *cnt, int plus, unsigned long long *sum) {
   const int tid = threadIdx.x;
@@ -143,7 +143,7 @@ __device__ __forceinline__ void finish_unit(const UnitLds &L, const uint32_t *__
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if ((tid & 63) == 0 && c) atomicAdd(sum, static_cast<unsigned long long>(c));
+  if ((tid & 63) == 0 && c) atomicAdd(accflat::sum_part(sum), static_cast<unsigned long long>(c));
 }
 
 // The probe of upper slot j: N(v) for v = adj[j] (empty for an id out of range).
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(kWG) void k_edge_wave(const uint32_t *__restrict__ 
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if (lane == 0 && c) atomicAdd(sum, static_cast<unsigned long long>(c));
+  if (lane == 0 && c) atomicAdd(accflat::sum_part(sum), static_cast<unsigned long long>(c));
 }
 
 // ---------------------------------------------------------------- BITMAP path
@@ -573,7 +573,7 @@ __global__ __launch_bounds__(kWG, 8) void k_bmp_lds(const uint32_t *__restrict__
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
-  if (lane == 0 && total) atomicAdd(sum, total);
+  if (lane == 0 && total) atomicAdd(accflat::sum_part(sum), total);
 }
 
 // ---------------------------------------------------------------- MERGE path
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(kWG) void k_merge_win(const uint32_t *__restrict__ 
 }
 
 __global__ void k_zero_sum(unsigned long long *sum) {
-  if (threadIdx.x == 0) *sum = 0;
+  sum[threadIdx.x * accfwd::kSumStride] = 0;
 }
 
 template <class K, class... A>
@@ -644,23 +644,23 @@ namespace accpaths {
 int launch_bitmap(acc_graph *g, int plus) {
   hipStream_t st = g->ctx->stream;
   const EdgePlan &p = g->edge;
-  hipLaunchKernelGGL(k_zero_sum, dim3(1), dim3(64), 0, st, g->d_sum);
+  hipLaunchKernelGGL(k_zero_sum, dim3(1), dim3(accfwd::kSumParts), 0, st, accfwd::sum_parts(g));
   ACC_HIP_TRY(hipGetLastError());
   ACC_TRY(launch_units(k_edge_wave<false>, (p.n_units[kEdgeWave] + kWaves - 1) / kWaves, st, g->d_off, g->d_adj,
-                       g->d_rev, g->n, p.d_units[kEdgeWave], p.n_units[kEdgeWave], g->d_cnt, plus, g->d_sum));
+                       g->d_rev, g->n, p.d_units[kEdgeWave], p.n_units[kEdgeWave], g->d_cnt, plus, accfwd::sum_parts(g)));
   ACC_TRY(launch_units(k_bmp_hash<12, true>, p.n_units[kEdgeHash12], st, g->d_off, g->d_adj, g->d_rev, g->n,
-                       p.d_units[kEdgeHash12], p.pool_words, p.idx_shift, g->d_cnt, plus, g->d_sum));
+                       p.d_units[kEdgeHash12], p.pool_words, p.idx_shift, g->d_cnt, plus, accfwd::sum_parts(g)));
   ACC_TRY(launch_units(k_bmp_hash<14, false>, p.n_units[kEdgeHash14], st, g->d_off, g->d_adj, g->d_rev, g->n,
-                       p.d_units[kEdgeHash14], p.pool_words, p.idx_shift, g->d_cnt, plus, g->d_sum));
+                       p.d_units[kEdgeHash14], p.pool_words, p.idx_shift, g->d_cnt, plus, accfwd::sum_parts(g)));
   ACC_TRY(launch_units(k_bmp_hash<15, false>, p.n_units[kEdgeHash15], st, g->d_off, g->d_adj, g->d_rev, g->n,
-                       p.d_units[kEdgeHash15], p.pool_words, p.idx_shift, g->d_cnt, plus, g->d_sum));
+                       p.d_units[kEdgeHash15], p.pool_words, p.idx_shift, g->d_cnt, plus, accfwd::sum_parts(g)));
   if (hubs_in_lds(g)) {
     const uint32_t words = static_cast<uint32_t>((p.pool_words + 3) & ~3ull);
     const uint32_t k = p.n_units[kEdgeHub];
     if (!k) return ACC_OK;
     const uint32_t grid = std::min<uint32_t>(k, 16 * std::max(1, g->ctx->num_cus));
     hipLaunchKernelGGL(k_bmp_lds<kU / 2>, dim3(grid), dim3(kWG), sizeof(LdsBitUnit) + 4 * words, st,
-                       g->d_off, g->d_adj, g->d_rev, g->n, p.d_units[kEdgeHub], k, words, g->d_cnt, plus, g->d_sum);
+                       g->d_off, g->d_adj, g->d_rev, g->n, p.d_units[kEdgeHub], k, words, g->d_cnt, plus, accfwd::sum_parts(g));
     ACC_HIP_TRY(hipGetLastError());
     return ACC_OK;
   }
@@ -673,7 +673,7 @@ int launch_bitmap(acc_graph *g, int plus) {
                        p.pool_words, true);
     ACC_HIP_TRY(hipGetLastError());
     ACC_TRY(launch_units(k_bmp_hub, u1 - u0, st, g->d_off, g->d_adj, g->d_rev, g->n, p.d_units[kEdgeHub] + u0,
-                         p.d_pool, p.pool_words, p.hub_idx_shift, g->d_cnt, plus, g->d_sum));
+                         p.d_pool, p.pool_words, p.hub_idx_shift, g->d_cnt, plus, accfwd::sum_parts(g)));
     hipLaunchKernelGGL(k_hub_bits, dim3(h1 - h0), dim3(256), 0, st, g->d_off, g->d_adj, p.d_hubs + h0, p.d_pool,
                        p.pool_words, false);
     ACC_HIP_TRY(hipGetLastError());
@@ -684,17 +684,17 @@ int launch_bitmap(acc_graph *g, int plus) {
 int launch_merge(acc_graph *g, int plus) {
   hipStream_t st = g->ctx->stream;
   const EdgePlan &p = g->edge;
-  hipLaunchKernelGGL(k_zero_sum, dim3(1), dim3(64), 0, st, g->d_sum);
+  hipLaunchKernelGGL(k_zero_sum, dim3(1), dim3(accfwd::kSumParts), 0, st, accfwd::sum_parts(g));
   ACC_HIP_TRY(hipGetLastError());
   ACC_TRY(launch_units(k_edge_wave<true>, (p.n_units[kEdgeWave] + kWaves - 1) / kWaves, st, g->d_off, g->d_adj,
-                       g->d_rev, g->n, p.d_units[kEdgeWave], p.n_units[kEdgeWave], g->d_cnt, plus, g->d_sum));
+                       g->d_rev, g->n, p.d_units[kEdgeWave], p.n_units[kEdgeWave], g->d_cnt, plus, accfwd::sum_parts(g)));
   // d_u <= 2048: one window of 2048 ids; the rest: windows of 8192 ids (38 KB
   // of LDS: four 512-thread workgroups per CU)
   ACC_TRY(launch_units(k_merge_win<11, kU>, p.n_units[kEdgeHash12], st, g->d_off, g->d_adj, g->d_rev, g->n,
-                       p.d_units[kEdgeHash12], g->d_cnt, plus, g->d_sum));
+                       p.d_units[kEdgeHash12], g->d_cnt, plus, accfwd::sum_parts(g)));
   for (int c : {kEdgeHash14, kEdgeHash15, kEdgeHub})
     ACC_TRY(launch_units(k_merge_win<13, kMergeU>, p.n_units[c], st, g->d_off, g->d_adj, g->d_rev, g->n, p.d_units[c],
-                         g->d_cnt, plus, g->d_sum));
+                         g->d_cnt, plus, accfwd::sum_parts(g)));
   return ACC_OK;
 }
 
