@@ -48,8 +48,10 @@ struct CopyLane {
 // hipMalloc and a hipFree take 30 and 40 us, and an upload with a SCAN query
 // made some 40 of each: 2.8 of its 7.6 ms at 262,144 vertices and 7.3M slots.
 // A block is reused without waiting: whoever frees one has waited for the
-// work that uses it, or that work and every later use are ordered by the
-// context's stream.  Safe from several threads.
+// work that uses it, or that work is queued on the context's stream.  So a block
+// used on another stream is not touched there before that stream has waited for
+// an event recorded on the context's stream after the alloc.  Safe from several
+// threads.
 class DevicePool {
  public:
   hipError_t alloc(void **p, size_t bytes);

@@ -1224,6 +1224,14 @@ int acc_scan_pairs(acc_scan_ws *w, int32_t *pairs, uint64_t cap, uint64_t *count
       w->d_pairs = nullptr;
       return acc_set_error(ACC_ENOMEM, "hipMalloc of the pair buffer failed");
     }
+    // the block's last use may still be queued on the context's stream (DevicePool)
+    hipError_t e = hipEventRecord(w->ready, g->ctx->stream);
+    if (e == hipSuccess) e = hipStreamWaitEvent(s, w->ready, 0);
+    if (e != hipSuccess) {
+      g->ctx->pool.free(w->d_pairs);
+      w->d_pairs = nullptr;
+      return acc_set_error(ACC_EDEVICE, std::string("pair buffer: ") + hipGetErrorString(e));
+    }
     w->device_bytes += bytes;
     w->pairs_cap = g->m;
   }
