@@ -312,7 +312,9 @@ struct ScanBuffers {
   uint32_t n_cap = 0;
   uint64_t m_cap = 0;
   uint64_t bytes = 0;
-  DevicePool *pool = nullptr;  // where the buffers come from (NULL: hipMalloc)
+  DevicePool *pool = nullptr;  // the context's
+  bool pooled = false;         // the buffers come from the pool, else from hipMalloc (the pool then
+                               // gives its idle blocks back where that fails)
 };
 
 namespace accscan {

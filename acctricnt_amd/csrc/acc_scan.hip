@@ -987,13 +987,15 @@ void free_buffers(ScanBuffers *b) {
                   static_cast<void *>(b->label),
                   static_cast<void *>(b->parent), static_cast<void *>(b->rmin), static_cast<void *>(b->rmax),
                   static_cast<void *>(b->cl), static_cast<void *>(b->cid), static_cast<void *>(b->counters)})
-    if (b->pool)
+    if (b->pooled)
       b->pool->free(p);
     else if (p)
       (void)hipFree(p);
   DevicePool *const pool = b->pool;
+  const bool pooled = b->pooled;
   *b = ScanBuffers{};
   b->pool = pool;
+  b->pooled = pooled;
 }
 
 // Grows the per-query buffers to hold a graph of n vertices and m slots.
@@ -1006,7 +1008,13 @@ int reserve_buffers(ScanBuffers *b, uint32_t n, uint64_t m) {
     using T = std::remove_pointer_t<std::remove_reference_t<decltype(*p)>>;
     const size_t bytes = sizeof(T) * (count ? count : 1);
     void **const to = reinterpret_cast<void **>(p);
-    if ((b->pool ? b->pool->alloc(to, bytes) : hipMalloc(to, bytes)) != hipSuccess) {
+    hipError_t e = b->pooled ? b->pool->alloc(to, bytes) : hipMalloc(to, bytes);
+    if (e != hipSuccess && !b->pooled && b->pool) {  // the idle blocks of the context may be what is in the way
+      (void)hipGetLastError();
+      b->pool->trim();
+      e = hipMalloc(to, bytes);
+    }
+    if (e != hipSuccess) {
       *p = nullptr;
       return acc_set_error(ACC_ENOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes of SCAN buffers failed");
     }
@@ -1141,6 +1149,7 @@ int acc_scan_ws_create(acc_graph *g, acc_scan_ws **out) {
   e = hipEventCreateWithFlags(&w->ready, hipEventDisableTiming);
   if (e != hipSuccess) return bail(acc_set_error(ACC_EDEVICE, std::string("hipEventCreate: ") + hipGetErrorString(e)));
   w->buf.pool = &g->ctx->pool;
+  w->buf.pooled = true;
   if ((rc = accscan::reserve_buffers(&w->buf, g->n, g->m))) return bail(rc);
   w->device_bytes = w->buf.bytes;
   if ((rc = acc_graph_ensure_src(g))) return bail(rc);

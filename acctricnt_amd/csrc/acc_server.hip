@@ -62,6 +62,7 @@ class HipDevice final : public accserve::Device {
  public:
   HipDevice(acc_ctx *ctx, const acc_server_config &cfg) : ctx_(ctx), no_index_(cfg.no_index != 0) {
     slots_.resize(static_cast<size_t>(cfg.slots));
+    for (Slot &sl : slots_) sl.buf.pool = &ctx->pool;
     streams_.resize(static_cast<size_t>(cfg.streams));
   }
   ~HipDevice() override {

@@ -68,3 +68,16 @@ def test_pairs_wait_for_the_context_stream(run):
         waits = [i for i, c in enumerate(calls) if c[0] == "wait"]
         assert all(t < max(waits) for t in taken), calls
     """)
+
+
+def test_result_slots_take_what_the_pool_holds_idle(run):
+    """Freed blocks of the context's graphs are kept for its next ones; where the
+    device has no more memory, a serving result slot gets it back from them."""
+    run("""
+    with cn.Context(0) as ctx:
+        ctx.upload(edgeless(1200000)).release()  # leaves blocks far larger than any below
+        with serve.Server(ctx, slots=1, streams=1) as sv:
+            # room for the graph (1.3 MB at most), not for its result slot (4.4 MB)
+            fake.fake_limit(fake.fake_held() + 2500000)
+            sv.query(sv.add_graph(edgeless(100000)), "0.5", 2)
+    """)
