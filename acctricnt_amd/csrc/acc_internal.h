@@ -57,6 +57,7 @@ class DevicePool {
   hipError_t alloc(void **p, size_t bytes);
   void free(void *p);
   void trim();
+  uint64_t idle_bytes();
   ~DevicePool() { trim(); }
 
  private:

@@ -528,6 +528,11 @@ void DevicePool::trim() {
   give_back(0);
 }
 
+uint64_t DevicePool::idle_bytes() {
+  std::lock_guard<std::mutex> lk(mu_);
+  return idle_bytes_;
+}
+
 void DevicePool::give_back(size_t most) {
   while (idle_bytes_ > most) {
     const auto last = std::prev(idle_.end());

@@ -110,6 +110,8 @@ class HipDevice final : public accserve::Device {
     return ACC_OK;
   }
   void release(void *handle) override { acc_graph_release(static_cast<acc_graph *>(handle)); }
+  uint64_t idle_bytes() override { return ctx_->pool.idle_bytes(); }
+  void drop_idle() override { ctx_->pool.trim(); }
 
   uint64_t slot_growth(int k, uint32_t n, uint64_t m) override {
     const Slot &sl = slots_[k];

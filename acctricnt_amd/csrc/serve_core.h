@@ -65,6 +65,10 @@ class Device {
   virtual int upload(uint32_t n, uint64_t m, const uint32_t *off, const int32_t *adj, bool validated, void **handle,
                      uint64_t *bytes) = 0;
   virtual void release(void *handle) = 0;
+  // Device bytes kept of released graphs and of uploads' scratch for later
+  // uploads, and giving them back to the device.  They count against the budget.
+  virtual uint64_t idle_bytes() { return 0; }
+  virtual void drop_idle() {}
   // Device bytes result slot k must add to hold a query on (n, m); 0 when it fits.
   virtual uint64_t slot_growth(int k, uint32_t n, uint64_t m) = 0;
   // Grows slot k for (n, m); *added = the device bytes it added (also on failure).
@@ -353,16 +357,20 @@ class Core {
     std::thread waiter;
   };
 
-  // Device bytes the budget still has room for.
-  uint64_t room() const {
+  // Whether `need` more bytes fit the budget beside the resident graphs and the
+  // result slots; idle bytes that would then exceed it go back to the device.
+  bool fits(uint64_t need) {
     const uint64_t used = graph_bytes_ + slot_bytes_;
-    return used >= cfg_.hbm_budget ? 0 : cfg_.hbm_budget - used;
+    const uint64_t room = used >= cfg_.hbm_budget ? 0 : cfg_.hbm_budget - used;
+    if (need > room) return false;
+    if (dev_->idle_bytes() > room - need) dev_->drop_idle();
+    return true;
   }
 
   // Evicts least recently used resident graphs with no running or pending
   // query (other than `keep`) until `need` bytes fit.  Caller holds mu_.
   bool make_room(uint64_t need, int32_t keep) {
-    while (room() < need) {
+    while (!fits(need)) {
       ServedGraph *victim = nullptr;
       for (auto &kv : graphs_) {
         ServedGraph &sg = kv.second;
@@ -404,12 +412,14 @@ class Core {
     graph_bytes_ -= need;
     if (rc) {
       sg.bytes = 0;
+      (void)fits(0);
       return rc;
     }
     sg.g = handle;
     sg.validated = true;
     sg.bytes = actual;
     graph_bytes_ += actual;
+    (void)fits(0);  // the upload's scratch is idle now
     st_.admissions++;
     return ACC_OK;
   }
@@ -418,7 +428,7 @@ class Core {
   // graphs for room when may_evict.  Caller holds mu_.
   int reserve_slot(int k, uint32_t n, uint64_t m, bool may_evict) {
     const uint64_t need = dev_->slot_growth(k, n, m);
-    if (need && (may_evict ? !make_room(need, -1) : room() < need))
+    if (need && !(may_evict ? make_room(need, -1) : fits(need)))
       return acc_set_error(ACC_EBUDGET, "no room for the result buffers of a query");
     uint64_t added = 0;
     const int rc = dev_->grow_slot(k, n, m, &added);

@@ -81,3 +81,18 @@ def test_result_slots_take_what_the_pool_holds_idle(run):
             fake.fake_limit(fake.fake_held() + 2500000)
             sv.query(sv.add_graph(edgeless(100000)), "0.5", 2)
     """)
+
+
+def test_serving_budget_counts_idle_blocks(run):
+    """hbm_budget bounds the device memory of a server's graphs, result slots and
+    what is kept of evicted graphs, whatever sizes came and went."""
+    run("""
+    budget = 25 << 20
+    with cn.Context(0) as ctx:
+        with serve.Server(ctx, hbm_budget=budget, slots=1, streams=1) as sv:
+            for n in (1000000, 860000, 740000, 630000, 540000, 460000, 390000, 330000, 280000):
+                sv.add_graph(edgeless(n))
+                assert fake.fake_held() <= budget, (n, fake.fake_held())
+            st = sv.stats()
+            assert st["evictions"] and fake.fake_held() >= st["graph_bytes"] + st["slot_bytes"]
+    """)
