@@ -156,6 +156,7 @@ struct DensePlan {
   uint32_t hit_cap = 0;           // most rows of a matrix that is kept
   uint64_t hit_bytes = 0;         // of all matrices
   uint8_t *d_hits = nullptr;      // allocated at the first per-slot pass
+  bool no_hits = false;           // ... which found no memory for them: every row is counted by atomics
   uint64_t bytes = 0, hits_held = 0;
   bool tables = false;            // d_vmeta, d_low and d_large match first and limit
 };
@@ -345,7 +346,8 @@ int build_tables(acc_graph *g);
 void free_tables(acc_graph *g);
 // What a pass needs, where the plan has dense units: the tables and, with
 // `slots`, the hit matrices (allocated once; zeroed where only a share's rows
-// are written).  Not under capture.
+// are written; passes count by atomics where there is no memory for them).
+// Not under capture.
 int ensure(acc_graph *g, bool slots);
 int clear_hits(acc_graph *g);
 int launch_count(acc_graph *g);

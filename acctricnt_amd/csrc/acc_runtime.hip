@@ -758,7 +758,7 @@ int acc_cn_compute(acc_graph *g, int path, uint32_t flags) {
     ACC_TRY(accfwd::launch_count_big(g));
     ACC_TRY(record(g, timing, "k_fwd_big"));
   }
-  if (g->dense.n_units) {
+  if (g->dense.n_units && g->dense.d_hits) {
     ACC_TRY(accdense::launch_rows(g));
     ACC_TRY(record(g, timing, "k_dense_rows"));
   }

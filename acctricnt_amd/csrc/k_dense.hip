@@ -24,8 +24,8 @@
 // triangle by a global atomic took most of the pass before.  The lower slots
 // then hold the complete counts and k_dense_gather copies them to the upper
 // slots.  Matrices of vertices with more than hit_cap dense neighbors are not
-// kept (their size grows with the square); their probes update the counts by
-// atomics.
+// kept (their size grows with the square), and none where the device has no
+// memory left for them; their probes update the counts by atomics.
 //
 // Measured at R-MAT scale 22 (4.2M vertices, 128M slots, 94% of 7.2e9 probe
 // elements at dense sources): counting 4.4 ms + 1.1 ms for the other sources
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kWG, 8) void k_dense(const uint4 *__restrict__ vmet
         len = (L + 7) >> 3;
         cb = mc.y;
         if (kSlots) {
-          direct = mc.z == kNoRows;
+          direct = !hits || mc.z == kNoRows;
           hb = direct ? 0 : mc.z + row_bytes(L);
         }
       }
@@ -700,6 +700,7 @@ void free_tables(acc_graph *g) {
   p.d_hits = nullptr;
   g->device_bytes -= p.bytes + p.hits_held;
   p.bytes = p.hits_held = 0;
+  p.no_hits = false;
   p.tables = false;
 }
 
@@ -794,11 +795,13 @@ int ensure(acc_graph *g, bool slots) {
   DensePlan &p = g->dense;
   if (!p.n_units) return ACC_OK;
   ACC_TRY(build_tables(g));
-  if (!slots || p.d_hits) return ACC_OK;
+  if (!slots || p.d_hits || p.no_hits) return ACC_OK;
   const uint64_t bytes = p.hit_bytes + 16;
   if (g->ctx->pool.alloc(reinterpret_cast<void **>(&p.d_hits), bytes) != hipSuccess) {
+    (void)hipGetLastError();
     p.d_hits = nullptr;
-    return acc_set_error(ACC_ENOMEM, "hipMalloc of the hit matrices failed");
+    p.no_hits = true;
+    return ACC_OK;
   }
   p.hits_held = bytes;
   g->device_bytes += bytes;
