@@ -169,8 +169,8 @@ void position_order(std::vector<FwdUnit> &units, const uint32_t *off, const uint
 
 // The dense sources of every graph (of the one graph without a partition):
 // their units within the shard, and the shard's other sources as ranges.
-// Tables made for other dense sources are dropped.
-void plan_dense(acc_graph *g, std::vector<FwdUnit> &units, std::vector<SourceRange> &rest) {
+// Tables made for other dense sources are dropped.  Without `dense` every graph has none.
+void plan_dense(acc_graph *g, bool dense, std::vector<FwdUnit> &units, std::vector<SourceRange> &rest) {
   DensePlan &p = g->dense;
   std::vector<uint32_t> first(1, 0), limit;
   if (g->num_parts) first.assign(g->h_gvoff.begin(), g->h_gvoff.end() - 1);
@@ -180,7 +180,7 @@ void plan_dense(acc_graph *g, std::vector<FwdUnit> &units, std::vector<SourceRan
   uint64_t upper = 0;
   for (size_t k = 0; k < first.size(); k++)
     limit.push_back(dense_sources(first[k], k + 1 < first.size() ? first[k + 1] : g->n, off, hs, &upper));
-  if (!accfwd::lower_counts(g) || upper < kDenseMin) std::fill(limit.begin(), limit.end(), 0u);
+  if (!dense || !accfwd::lower_counts(g) || upper < kDenseMin) std::fill(limit.begin(), limit.end(), 0u);
   for (size_t k = 0; k < first.size(); k++) {
     const uint32_t v0 = first[k];
     const uint32_t lo = std::max(v0, g->shard_lo), hi = std::min(v0 + limit[k], g->shard_hi);
@@ -201,13 +201,13 @@ void plan_dense(acc_graph *g, std::vector<FwdUnit> &units, std::vector<SourceRan
 }
 
 // Rebuilds the forward plan from the host split points, the current bin
-// parameters and the shard; the per-edge plans are rebuilt at their next use.
-int upload_plans(acc_graph *g) {
+// parameters and the shard, with dense sources or without.
+int upload_forward(acc_graph *g, bool with_dense) {
   drop_capture(g);
   std::vector<FwdUnit> wave, block, big, dense;
   const uint32_t device_waves = static_cast<uint32_t>(std::max(1, g->ctx->num_cus)) * 32u;
   std::vector<SourceRange> ranges;
-  plan_dense(g, dense, ranges);
+  plan_dense(g, with_dense, dense, ranges);
   build_forward_plan(ranges, g->h_off.data(), g->h_hs.data(), g->h_lo.data(), g->wave_slots,
                      g->wave_low, g->chunk, device_waves, wave, block, big);
   // Workgroup units in a stride order (the golden-ratio stride, coprime with
@@ -226,10 +226,19 @@ int upload_plans(acc_graph *g) {
                       {&block, &g->d_fwd_block, &g->n_fwd_block},
                       {&big, &g->d_fwd_big, &g->n_fwd_big},
                       {&dense, &g->dense.d_units, &g->dense.n_units}};
-  g->edge.valid = false;
   ACC_TRY(upload_lists(g, lists));
   ACC_TRY(accdense::ensure(g, false));
   return accdense::clear_hits(g);
+}
+
+// Rebuilds the forward plan; the per-edge plans are rebuilt at their next use.
+// Dense sources only save time, so where the device has no memory for their
+// tables the plan goes without.
+int upload_plans(acc_graph *g) {
+  g->edge.valid = false;
+  int rc = upload_forward(g, true);
+  if (rc == ACC_ENOMEM && g->dense.n_units) rc = upload_forward(g, false);
+  return rc;
 }
 
 // The per-edge (bitmap and merge) plans, built at the first pass that needs

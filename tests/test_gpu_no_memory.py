@@ -1,6 +1,6 @@
 """Counting with dense sources where the device has no memory for what only
-makes it faster: the hit matrices at the first per-slot pass.  hipMalloc of
-that size fails on demand (tests/hip_host/fail_alloc.cpp) in a process of its
+makes it faster: the hit matrices at the first per-slot pass, and the tables at
+the upload.  hipMalloc of that size fails on demand (tests/hip_host/fail_alloc.cpp) in a process of its
 own, and every count and total equals the oracle's."""
 import os
 import subprocess
@@ -41,6 +41,7 @@ def check(rg):
         acc += cnt
         tri += t
     assert np.array_equal(acc, ref - 2) and tri == total
+    rg.set_shard(1, 0)
 """
 
 
@@ -69,6 +70,19 @@ def test_without_hit_matrices(run):
         check(rg)
         assert fail.fail_alloc_failed() > 0
         fail.fail_alloc_between(1, 0)
-        rg.set_shard(1, 0)
         check(rg)
+    """)
+
+
+def test_without_tables(run):
+    run("""
+    for size in (16 * g.n, 24 * g.n):  # the vertex records, the tables' scratch
+        with cn.Context(0) as ctx:
+            fail.fail_alloc_between(size, size + (size >> 2) + (64 << 10))
+            with ctx.upload(g) as rg:
+                assert fail.fail_alloc_failed() > 0
+                fail.fail_alloc_between(1, 0)
+                check(rg)
+                rg.set_param("chunk", 256)  # the next plan finds memory
+                check(rg)
     """)
