@@ -158,6 +158,7 @@ struct DensePlan {
   uint8_t *d_hits = nullptr;      // allocated at the first per-slot pass
   bool no_hits = false;           // ... which found no memory for them: every row is counted by atomics
   uint64_t bytes = 0, hits_held = 0;
+  bool allowed = true;            // the plan may have dense sources
   bool tables = false;            // d_vmeta, d_low and d_large match first and limit
 };
 
@@ -245,6 +246,10 @@ inline bool hubs_in_lds(const acc_graph *g) { return g->n <= kLdsBitmapIds; }
 int launch_bitmap(acc_graph *g, int plus);
 int launch_merge(acc_graph *g, int plus);
 }  // namespace accpaths
+
+// acc_graph_upload, with dense sources or without (acc_runtime.hip).
+int acc_upload(acc_ctx *ctx, uint32_t n, uint64_t m, const uint32_t *node_off, const int32_t *edge_dst, uint32_t flags,
+               bool dense, acc_graph **out);
 
 // Builds the slot -> source array (acc_scan.hip).
 int acc_graph_ensure_src(acc_graph *g);
@@ -341,6 +346,11 @@ int launch_index_jobs(const JobTable &jt, uint32_t vblocks, uint32_t sblocks, hi
 // Dense sources (k_dense.hip).
 namespace accdense {
 constexpr uint32_t kMaxRows = 4096;  // most rows of a hit matrix that is kept
+// Most bytes of a graph's hit matrices: 32-bit offsets, 16 bytes per slot.
+inline uint64_t most_hit_bytes(uint64_t m) {
+  const uint64_t by_slots = 16 * m + (1u << 20);
+  return by_slots < 0xe0000000ull ? by_slots : 0xe0000000ull;
+}
 // The vertex records, low lists and matrix offsets for dense.first / limit.
 int build_tables(acc_graph *g);
 void free_tables(acc_graph *g);

@@ -180,7 +180,7 @@ void plan_dense(acc_graph *g, bool dense, std::vector<FwdUnit> &units, std::vect
   uint64_t upper = 0;
   for (size_t k = 0; k < first.size(); k++)
     limit.push_back(dense_sources(first[k], k + 1 < first.size() ? first[k + 1] : g->n, off, hs, &upper));
-  if (!dense || !accfwd::lower_counts(g) || upper < kDenseMin) std::fill(limit.begin(), limit.end(), 0u);
+  if (!dense || !p.allowed || !accfwd::lower_counts(g) || upper < kDenseMin) std::fill(limit.begin(), limit.end(), 0u);
   for (size_t k = 0; k < first.size(); k++) {
     const uint32_t v0 = first[k];
     const uint32_t lo = std::max(v0, g->shard_lo), hi = std::min(v0 + limit[k], g->shard_hi);
@@ -557,6 +557,70 @@ int acc_set_error(int code, const std::string &msg) {
   return code;
 }
 
+int acc_upload(acc_ctx *ctx, uint32_t n, uint64_t m, const uint32_t *node_off, const int32_t *edge_dst, uint32_t flags,
+               bool dense, acc_graph **out) {
+  if (!ctx || !out || !node_off || (m && !edge_dst)) return acc_set_error(ACC_EINVAL, "null argument");
+  *out = nullptr;
+  if (flags & ~(ACC_UPLOAD_NO_VALIDATE | ACC_UPLOAD_RELABEL))
+    return acc_set_error(ACC_EINVAL, "unknown upload flags " + std::to_string(flags));
+  if (m >= (1ULL << 32)) return acc_set_error(ACC_EINVAL, "m must be below 2^32 (uint32 node_off)");
+  if (n >= (1u << 31)) return acc_set_error(ACC_EINVAL, "n must be below 2^31 (int32 ids)");
+  if (node_off[0] != 0 || node_off[n] != m) return acc_set_error(ACC_EFORMAT, "node_off[0] != 0 or node_off[n] != m");
+  for (uint32_t u = 0; u < n; u++)
+    if (node_off[u + 1] < node_off[u])
+      return acc_set_error(ACC_EFORMAT, "node_off not monotone at vertex " + std::to_string(u));
+  DeviceGuard guard(ctx->device);
+  auto *g = new (std::nothrow) acc_graph;
+  if (!g) return acc_set_error(ACC_ENOMEM, "host allocation failed");
+  g->ctx = ctx;
+  g->n = n;
+  g->m = m;
+  g->shard_hi = n;
+  g->dense.allowed = dense;
+  int rc = ACC_OK;
+  auto bail = [&](int code) {
+    free_graph(g);
+    return code;
+  };
+  if ((rc = dev_alloc(g, &g->d_off, static_cast<uint64_t>(n) + 1))) return bail(rc);
+  if ((rc = dev_alloc(g, &g->d_adj, m + kAdjPad))) return bail(rc);
+  if ((rc = dev_alloc(g, &g->d_cnt, m + 4))) return bail(rc);
+  if ((rc = dev_alloc(g, &g->d_rev, m + 4))) return bail(rc);
+  if ((rc = dev_alloc(g, &g->d_sum, accfwd::kSumStride * (1 + accfwd::kSumParts)))) return bail(rc);
+  if ((rc = dev_alloc(g, &g->d_flags, 4))) return bail(rc);
+  if ((rc = staged_copy(ctx, g->d_off, node_off, sizeof(uint32_t) * (static_cast<size_t>(n) + 1), true)))
+    return bail(rc);
+  if ((rc = staged_copy(ctx, g->d_adj, edge_dst, sizeof(int32_t) * m, true))) return bail(rc);
+  hipError_t e = hipMemsetAsync(g->d_flags, 0, sizeof(int32_t) * 4, ctx->stream);
+  if (e != hipSuccess) return bail(acc_set_error(ACC_EDEVICE, std::string("upload: ") + hipGetErrorString(e)));
+  const bool relabel = (flags & ACC_UPLOAD_RELABEL) != 0;
+  const bool validate = !(flags & ACC_UPLOAD_NO_VALIDATE) || relabel;  // the relabel indexes by neighbor id
+  int32_t hf[4] = {0, 0, 0, 0};
+  auto read_flags = [&]() {
+    hipError_t err = hipMemcpyAsync(hf, g->d_flags, sizeof(hf), hipMemcpyDeviceToHost, ctx->stream);
+    if (err == hipSuccess) err = hipStreamSynchronize(ctx->stream);
+    return err == hipSuccess ? ACC_OK
+                             : acc_set_error(ACC_EDEVICE, std::string("validate: ") + hipGetErrorString(err));
+  };
+  if ((rc = accprep::slot_sources(g))) return bail(rc);
+  if (validate) {
+    if ((rc = accfwd::launch_validate(g)) || (rc = read_flags())) return bail(rc);
+    if (hf[0] & 1) return bail(acc_set_error(ACC_EFORMAT, "neighbor id out of range"));
+    if (hf[0] & 2) return bail(acc_set_error(ACC_EFORMAT, "Self loop"));
+    if (hf[0] & 4) return bail(acc_set_error(ACC_EFORMAT, "Edges not sorted in increasing id order"));
+  }
+  if (relabel && ((rc = accprep::relabel_degree(g)) || (rc = accprep::slot_sources(g)))) return bail(rc);
+  if ((rc = load_vertex_meta(g, relabel ? nullptr : node_off))) return bail(rc);
+  uint64_t upper = 0;
+  if ((rc = accprep::reverse_slots(g, validate, &upper))) return bail(rc);
+  if ((rc = read_flags())) return bail(rc);
+  g->symmetric = !(hf[0] & 8) && 2 * upper == m;
+  if (validate && !g->symmetric) return bail(acc_set_error(ACC_EFORMAT, "CSR not symmetric"));
+  if ((rc = upload_plans(g))) return bail(rc);
+  *out = g;
+  return ACC_OK;
+}
+
 extern "C" {
 
 const char *acc_last_error(void) { return g_err.c_str(); }
@@ -637,65 +701,7 @@ void *acc_ctx_stream(acc_ctx *ctx) { return ctx ? static_cast<void *>(ctx->strea
 
 int acc_graph_upload(acc_ctx *ctx, uint32_t n, uint64_t m, const uint32_t *node_off, const int32_t *edge_dst,
                      uint32_t flags, acc_graph **out) {
-  if (!ctx || !out || !node_off || (m && !edge_dst)) return acc_set_error(ACC_EINVAL, "null argument");
-  *out = nullptr;
-  if (flags & ~(ACC_UPLOAD_NO_VALIDATE | ACC_UPLOAD_RELABEL))
-    return acc_set_error(ACC_EINVAL, "unknown upload flags " + std::to_string(flags));
-  if (m >= (1ULL << 32)) return acc_set_error(ACC_EINVAL, "m must be below 2^32 (uint32 node_off)");
-  if (n >= (1u << 31)) return acc_set_error(ACC_EINVAL, "n must be below 2^31 (int32 ids)");
-  if (node_off[0] != 0 || node_off[n] != m) return acc_set_error(ACC_EFORMAT, "node_off[0] != 0 or node_off[n] != m");
-  for (uint32_t u = 0; u < n; u++)
-    if (node_off[u + 1] < node_off[u])
-      return acc_set_error(ACC_EFORMAT, "node_off not monotone at vertex " + std::to_string(u));
-  DeviceGuard guard(ctx->device);
-  auto *g = new (std::nothrow) acc_graph;
-  if (!g) return acc_set_error(ACC_ENOMEM, "host allocation failed");
-  g->ctx = ctx;
-  g->n = n;
-  g->m = m;
-  g->shard_hi = n;
-  int rc = ACC_OK;
-  auto bail = [&](int code) {
-    free_graph(g);
-    return code;
-  };
-  if ((rc = dev_alloc(g, &g->d_off, static_cast<uint64_t>(n) + 1))) return bail(rc);
-  if ((rc = dev_alloc(g, &g->d_adj, m + kAdjPad))) return bail(rc);
-  if ((rc = dev_alloc(g, &g->d_cnt, m + 4))) return bail(rc);
-  if ((rc = dev_alloc(g, &g->d_rev, m + 4))) return bail(rc);
-  if ((rc = dev_alloc(g, &g->d_sum, accfwd::kSumStride * (1 + accfwd::kSumParts)))) return bail(rc);
-  if ((rc = dev_alloc(g, &g->d_flags, 4))) return bail(rc);
-  if ((rc = staged_copy(ctx, g->d_off, node_off, sizeof(uint32_t) * (static_cast<size_t>(n) + 1), true)))
-    return bail(rc);
-  if ((rc = staged_copy(ctx, g->d_adj, edge_dst, sizeof(int32_t) * m, true))) return bail(rc);
-  hipError_t e = hipMemsetAsync(g->d_flags, 0, sizeof(int32_t) * 4, ctx->stream);
-  if (e != hipSuccess) return bail(acc_set_error(ACC_EDEVICE, std::string("upload: ") + hipGetErrorString(e)));
-  const bool relabel = (flags & ACC_UPLOAD_RELABEL) != 0;
-  const bool validate = !(flags & ACC_UPLOAD_NO_VALIDATE) || relabel;  // the relabel indexes by neighbor id
-  int32_t hf[4] = {0, 0, 0, 0};
-  auto read_flags = [&]() {
-    hipError_t err = hipMemcpyAsync(hf, g->d_flags, sizeof(hf), hipMemcpyDeviceToHost, ctx->stream);
-    if (err == hipSuccess) err = hipStreamSynchronize(ctx->stream);
-    return err == hipSuccess ? ACC_OK
-                             : acc_set_error(ACC_EDEVICE, std::string("validate: ") + hipGetErrorString(err));
-  };
-  if ((rc = accprep::slot_sources(g))) return bail(rc);
-  if (validate) {
-    if ((rc = accfwd::launch_validate(g)) || (rc = read_flags())) return bail(rc);
-    if (hf[0] & 1) return bail(acc_set_error(ACC_EFORMAT, "neighbor id out of range"));
-    if (hf[0] & 2) return bail(acc_set_error(ACC_EFORMAT, "Self loop"));
-    if (hf[0] & 4) return bail(acc_set_error(ACC_EFORMAT, "Edges not sorted in increasing id order"));
-  }
-  if (relabel && ((rc = accprep::relabel_degree(g)) || (rc = accprep::slot_sources(g)))) return bail(rc);
-  if ((rc = load_vertex_meta(g, relabel ? nullptr : node_off))) return bail(rc);
-  uint64_t upper = 0;
-  if ((rc = accprep::reverse_slots(g, validate, &upper))) return bail(rc);
-  if ((rc = read_flags())) return bail(rc);
-  g->symmetric = !(hf[0] & 8) && 2 * upper == m;
-  if (validate && !g->symmetric) return bail(acc_set_error(ACC_EFORMAT, "CSR not symmetric"));
-  if ((rc = upload_plans(g))) return bail(rc);
-  *out = g;
-  return ACC_OK;
+  return acc_upload(ctx, n, m, node_off, edge_dst, flags, true, out);
 }
 
 void acc_graph_release(acc_graph *g) { free_graph(g); }

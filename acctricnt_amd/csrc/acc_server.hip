@@ -50,6 +50,13 @@ uint64_t graph_estimate(uint32_t n, uint64_t m) {
          (1ull << 20);
 }
 
+// Most that the dense sources of the graph's one counting pass hold: the scratch,
+// records, lists and matrices of k_dense.hip.
+uint64_t dense_most(uint32_t n, uint64_t m) {
+  if (m < 2 * kDenseMin) return 0;  // too few upper slots for dense sources
+  return 76ull * (n + 1) + 3ull * m + accdense::most_hit_bytes(m) + (2ull << 20);
+}
+
 void free_slot(Slot &s) {
   accscan::free_buffers(&s.buf);
   if (s.h_label) (void)hipHostFree(s.h_label);
@@ -87,12 +94,15 @@ class HipDevice final : public accserve::Device {
   int check_query(int64_t p, int64_t q, int32_t) override { return accscan::check_eps(p, q); }
   uint64_t estimate(uint32_t n, uint64_t m) override { return graph_estimate(n, m); }
 
+  uint64_t upload_extra(uint32_t n, uint64_t m) override { return dense_most(n, m); }
+  void allow_extra(bool dense) override { dense_ = dense; }
+
   // Uploads the graph and computes its counts, slot sources and index
   // (serialised by the core; the upload takes milliseconds).
   int upload(uint32_t n, uint64_t m, const uint32_t *off, const int32_t *adj, bool validated, void **handle,
              uint64_t *bytes) override {
     acc_graph *g = nullptr;
-    int rc = acc_graph_upload(ctx_, n, m, off, adj, validated ? ACC_UPLOAD_NO_VALIDATE : 0u, &g);
+    int rc = acc_upload(ctx_, n, m, off, adj, validated ? ACC_UPLOAD_NO_VALIDATE : 0u, dense_, &g);
     if (!rc) rc = acc_cn_compute(g, ACC_PATH_AUTO, 0);
     if (!rc) rc = acc_graph_ensure_src(g);
     if (!rc) rc = acc_ctx_synchronize(ctx_);
@@ -228,6 +238,7 @@ class HipDevice final : public accserve::Device {
  private:
   acc_ctx *ctx_;
   bool no_index_;
+  bool dense_ = true;  // whether the next upload may use dense sources
   std::vector<Slot> slots_;
   std::vector<Stream> streams_;
 };

@@ -746,8 +746,8 @@ int build_tables(acc_graph *g) {
   }
   if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(temp, t_scan, wide, wide0, static_cast<int>(n1), st);
   if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(temp, t_scan, narrow, narrow0, static_cast<int>(n1), st);
-  // the largest cap whose matrices stay within 32-bit offsets and 16 bytes per slot
-  const uint64_t most = std::min<uint64_t>(0xe0000000ull, 16 * g->m + (1u << 20));
+  // the largest cap whose matrices stay within the limit
+  const uint64_t most = most_hit_bytes(g->m);
   DenseSizes h{};
   p.hit_cap = 2 * kMaxRows;
   do {

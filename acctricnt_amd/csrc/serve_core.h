@@ -64,6 +64,10 @@ class Device {
   // *handle and its actual footprint *bytes on success.
   virtual int upload(uint32_t n, uint64_t m, const uint32_t *off, const int32_t *adj, bool validated, void **handle,
                      uint64_t *bytes) = 0;
+  // Device bytes beyond the estimate that a faster upload holds until it
+  // returns, and whether the next upload may (a call before each).
+  virtual uint64_t upload_extra(uint32_t, uint64_t) { return 0; }
+  virtual void allow_extra(bool) {}
   virtual void release(void *handle) = 0;
   // Device bytes kept of released graphs and of uploads' scratch for later
   // uploads, and giving them back to the device.  They count against the budget.
@@ -399,12 +403,16 @@ class Core {
     graph_bytes_ += need;
     sg.bytes = need;
     sg.running++;  // pins the entry against eviction and removal while unlocked
+    // Nothing is evicted for the extra and it is not reserved: queries launched
+    // meanwhile may grow their slots.
+    const bool extra = fits(dev_->upload_extra(sg.n, sg.m));
     lk.unlock();
     int rc;
     void *handle = nullptr;
     uint64_t actual = 0;
     {
       std::lock_guard<std::mutex> ag(admit_mu_);
+      dev_->allow_extra(extra);
       rc = dev_->upload(sg.n, sg.m, sg.off.data(), sg.adj.data(), sg.validated, &handle, &actual);
     }
     lk.lock();

@@ -86,3 +86,25 @@ def test_without_tables(run):
                 rg.set_param("chunk", 256)  # the next plan finds memory
                 check(rg)
     """)
+
+
+def test_admission_within_the_budget(run):
+    """A served graph is counted with dense sources only where their tables and
+    matrices fit the server's budget beside it."""
+    run("""
+    from acctricnt_amd import serve
+    with cn.Context(0) as ctx, ctx.upload(g) as rg:
+        before = rg.device_bytes()
+        rg.compute("forward")
+        hits = rg.device_bytes() - before
+    ref_scan = oracle.scan(g, ref, "0.3", 5)
+    # the graph and one result slot: 28.3 and 1.1 bytes a slot, 20 and 45 a vertex
+    tight = 30 * g.m + 65 * g.n + (4 << 20)
+    for budget, asked in ((tight, False), (2 * tight, True)):
+        with cn.Context(0) as ctx, serve.Server(ctx, hbm_budget=budget, slots=1) as sv:
+            fail.fail_alloc_between(hits, hits + (64 << 10))
+            gid = sv.add_graph(g)
+            assert (fail.fail_alloc_failed() > 0) == asked
+            res = sv.query(gid, "0.3", 5)
+            assert np.array_equal(res["label"], ref_scan["label"])
+    """)
