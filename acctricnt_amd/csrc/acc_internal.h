@@ -117,7 +117,7 @@ int bind_scratch(int device, unsigned long long **addr);
 // sorted run.  Block units: the bitmap path keeps N(u) in an LDS hash table
 // of 2^12, 2^14 or 2^15 keys (d_u up to half of that) or, for hubs, in an HBM
 // bitmap; the merge path stages N(u) in LDS windows of 2^11 ids (the first
-// class) or 2^13 ids (the others).
+// class, and the units behind the hub units) or 2^13 ids (the others).
 enum EdgeClass { kEdgeWave = 0, kEdgeHash12, kEdgeHash14, kEdgeHash15, kEdgeHub, kEdgeClasses };
 constexpr uint32_t kEdgeWaveDeg = 256;  // d_u of a wave unit
 constexpr int kEdgeWaveLog = 8;         // log2 kEdgeWaveDeg
@@ -126,6 +126,7 @@ constexpr uint32_t kEdgeWaveUp = 64;    // upper slots of a wave unit
 struct EdgePlan {
   FwdUnit *d_units[kEdgeClasses] = {};  // hub units: nlow = the hub's bitmap in its batch's pool
   uint32_t n_units[kEdgeClasses] = {};
+  uint32_t n_small = 0;                 // units with d_u <= 256 behind the hub units, where hub bitmaps lie in LDS
   uint32_t *d_hubs = nullptr;           // hub sources in order
   uint32_t n_hubs = 0;
   std::vector<uint32_t> hub_batch;       // batch k: hubs [hub_batch[k], hub_batch[k+1])

@@ -61,24 +61,27 @@ void free_graph(acc_graph *g) {
 // 8192 and min(16384, hash_max); the rest are hubs.  Hubs go into batches of at
 // most pool_hubs (one HBM bitmap each); a hub unit's nlow is its hub's
 // bitmap within the batch.  Where hub bitmaps lie in LDS (lds_hubs), the
-// smallest block units, d_u <= 256, are hubs too.
+// smallest block units, d_u <= min(256, hash_max), follow the hub units (n_small of
+// them), for the bitmap path to run both alike and the merge path each as the others of its length.
 constexpr uint64_t kHubPoolBytes = 8ull << 30;  // HBM bitmaps of one hub batch
 constexpr uint32_t kHubBatch = 16384;           // most hubs of one batch (ACC_PARAM_BMP_BATCH)
 constexpr uint32_t kHashIdxBits = 1u << 17;     // LDS index bits of a hash unit (k_bmp_hash's kIdxWords)
 constexpr uint32_t kHubIdxBits = 1u << 18;      // LDS index bits of a hub unit (k_bmp_hub's kHubIdxWords)
 void build_edge_plan(uint32_t n, const uint32_t *off, const uint32_t *hs, uint32_t chunk, uint32_t hash_max,
                      uint32_t pool_hubs, bool lds_hubs, std::vector<FwdUnit> (&units)[kEdgeClasses], std::vector<uint32_t> &hubs,
-                     std::vector<uint32_t> &hub_batch, std::vector<uint32_t> &hub_unit_batch) {
+                     std::vector<uint32_t> &hub_batch, std::vector<uint32_t> &hub_unit_batch, uint32_t &n_small) {
   hub_batch.assign(1, 0);
   hub_unit_batch.assign(1, 0);
+  std::vector<FwdUnit> small;
   for (uint32_t u = 0; u < n; u++) {
     const uint32_t du = off[u + 1] - off[u];
     if (hs[u] == off[u + 1]) continue;
     int c = kEdgeHub;
     if (du <= kEdgeWaveDeg && off[u + 1] - hs[u] <= kEdgeWaveUp)
       c = kEdgeWave;
-    else if (du <= hash_max && !(lds_hubs && du <= kEdgeWaveDeg))
+    else if (du <= hash_max)
       c = du <= 2048 ? kEdgeHash12 : du <= 8192 ? kEdgeHash14 : kEdgeHash15;
+    std::vector<FwdUnit> &to = lds_hubs && c == kEdgeHash12 && du <= kEdgeWaveDeg ? small : units[c];
     uint32_t slot = 0;
     if (c == kEdgeHub) {
       if (hubs.size() - hub_batch.back() == pool_hubs) {
@@ -89,10 +92,12 @@ void build_edge_plan(uint32_t n, const uint32_t *off, const uint32_t *hs, uint32
       hubs.push_back(u);
     }
     for (uint32_t j0 = hs[u]; j0 < off[u + 1]; j0 += chunk)
-      units[c].push_back(FwdUnit{static_cast<int32_t>(u), j0, std::min(j0 + chunk, off[u + 1]), c == kEdgeHub ? slot : du});
+      to.push_back(FwdUnit{static_cast<int32_t>(u), j0, std::min(j0 + chunk, off[u + 1]), c == kEdgeHub ? slot : du});
   }
   hub_batch.push_back(static_cast<uint32_t>(hubs.size()));
   hub_unit_batch.push_back(static_cast<uint32_t>(units[kEdgeHub].size()));
+  n_small = static_cast<uint32_t>(small.size());
+  units[kEdgeHub].insert(units[kEdgeHub].end(), small.begin(), small.end());
 }
 
 template <typename T>
@@ -257,7 +262,7 @@ int ensure_edge_plans(acc_graph *g) {
   std::vector<FwdUnit> units[kEdgeClasses];
   std::vector<uint32_t> hubs;
   build_edge_plan(g->n, g->h_off.data(), g->h_hs.data(), g->chunk, g->bmp_hash_max, pool_hubs, accpaths::hubs_in_lds(g), units, hubs,
-                  p.hub_batch, p.hub_unit_batch);
+                  p.hub_batch, p.hub_unit_batch, p.n_small);
   PlanList lists[] = {{&units[kEdgeWave], &p.d_units[kEdgeWave], &p.n_units[kEdgeWave]},
                       {&units[kEdgeHash12], &p.d_units[kEdgeHash12], &p.n_units[kEdgeHash12]},
                       {&units[kEdgeHash14], &p.d_units[kEdgeHash14], &p.n_units[kEdgeHash14]},

@@ -688,13 +688,16 @@ int launch_merge(acc_graph *g, int plus) {
   ACC_HIP_TRY(hipGetLastError());
   ACC_TRY(launch_units(k_edge_wave<true>, (p.n_units[kEdgeWave] + kWaves - 1) / kWaves, st, g->d_off, g->d_adj,
                        g->d_rev, g->n, p.d_units[kEdgeWave], p.n_units[kEdgeWave], g->d_cnt, plus, accfwd::sum_parts(g)));
-  // d_u <= 2048: one window of 2048 ids; the rest: windows of 8192 ids (38 KB
-  // of LDS: four 512-thread workgroups per CU)
+  // d_u <= min(2048, bmp_hash_max): one window of 2048 ids; the rest: windows of
+  // 8192 ids (38 KB of LDS: four 512-thread workgroups per CU)
+  const uint32_t hubs = p.n_units[kEdgeHub] - p.n_small;
   ACC_TRY(launch_units(k_merge_win<11, kU>, p.n_units[kEdgeHash12], st, g->d_off, g->d_adj, g->d_rev, g->n,
                        p.d_units[kEdgeHash12], g->d_cnt, plus, accfwd::sum_parts(g)));
+  ACC_TRY(launch_units(k_merge_win<11, kU>, p.n_small, st, g->d_off, g->d_adj, g->d_rev, g->n,
+                       p.d_units[kEdgeHub] + hubs, g->d_cnt, plus, accfwd::sum_parts(g)));
   for (int c : {kEdgeHash14, kEdgeHash15, kEdgeHub})
-    ACC_TRY(launch_units(k_merge_win<13, kMergeU>, p.n_units[c], st, g->d_off, g->d_adj, g->d_rev, g->n, p.d_units[c],
-                         g->d_cnt, plus, accfwd::sum_parts(g)));
+    ACC_TRY(launch_units(k_merge_win<13, kMergeU>, c == kEdgeHub ? hubs : p.n_units[c], st, g->d_off, g->d_adj,
+                         g->d_rev, g->n, p.d_units[c], g->d_cnt, plus, accfwd::sum_parts(g)));
   return ACC_OK;
 }
 

@@ -96,3 +96,24 @@ def test_serving_budget_counts_idle_blocks(run):
             st = sv.stats()
             assert st["evictions"] and fake.fake_held() >= st["graph_bytes"] + st["slot_bytes"]
     """)
+
+
+def test_merge_windows_of_small_units(run):
+    """Workgroup units with few neighbors take the merge path's small windows,
+    whatever the bitmap path makes of them."""
+    run("""
+    n, deg = 300, 100  # (trusted: every kernel does nothing, so nothing is checked)
+    off = np.arange(n + 1, dtype=np.uint32) * deg
+    g = CSRGraph(off, np.tile(np.arange(deg, dtype=np.int32), n))
+    with cn.Context(0) as ctx, ctx.upload(g, validate=False) as rg:
+        fake.fake_clear()
+        rg.compute("merge")
+        names = [c[2] for c in log() if c[0] == "launch"]
+        assert any("k_merge_winILi11E" in k for k in names), names
+        assert not any("k_merge_winILi13E" in k for k in names), names
+        fake.fake_clear()
+        rg.set_param("bmp_hash_max", 0)  # every workgroup unit a hub
+        rg.compute("merge")
+        names = [c[2] for c in log() if c[0] == "launch"]
+        assert any("k_merge_winILi13E" in k for k in names) and not any("k_merge_winILi11E" in k for k in names)
+    """)
