@@ -357,8 +357,8 @@ int build_tables(acc_graph *g);
 void free_tables(acc_graph *g);
 // What a pass needs, where the plan has dense units: the tables and, with
 // `slots`, the hit matrices (allocated once; zeroed where only a share's rows
-// are written; passes count by atomics where there is no memory for them).
-// Not under capture.
+// are written; passes count by atomics where there is no memory for them, or
+// where the stream is recorded before they are there).
 int ensure(acc_graph *g, bool slots);
 int clear_hits(acc_graph *g);
 int launch_count(acc_graph *g);

@@ -796,6 +796,10 @@ int ensure(acc_graph *g, bool slots) {
   if (!p.n_units) return ACC_OK;
   ACC_TRY(build_tables(g));
   if (!slots || p.d_hits || p.no_hits) return ACC_OK;
+  // a caller who records the stream gets a pass by atomics: nothing is allocated under it
+  hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+  ACC_HIP_TRY(hipStreamIsCapturing(g->ctx->stream, &recording));
+  if (recording != hipStreamCaptureStatusNone) return ACC_OK;
   const uint64_t bytes = p.hit_bytes + 16;
   if (g->ctx->pool.alloc(reinterpret_cast<void **>(&p.d_hits), bytes) != hipSuccess) {
     (void)hipGetLastError();
