@@ -521,19 +521,28 @@ hipError_t DevicePool::alloc(void **p, size_t bytes) {
     give_back(0);
     e = hipMalloc(p, bytes);
   }
-  if (e == hipSuccess)
-    size_[*p] = bytes;
-  else
-    *p = nullptr;
+  if (e == hipSuccess) try {
+      size_.emplace(*p, bytes);
+    } catch (const std::bad_alloc &) {
+      (void)hipFree(*p);
+      e = hipErrorOutOfMemory;
+    }
+  if (e != hipSuccess) *p = nullptr;
   return e;
 }
 
 void DevicePool::free(void *p) {
   if (!p) return;
   std::lock_guard<std::mutex> lk(mu_);
-  const size_t bytes = size_[p];
-  idle_.emplace(bytes, p);
-  idle_bytes_ += bytes;
+  const auto it = size_.find(p);
+  try {
+    idle_.emplace(it->second, p);
+  } catch (const std::bad_alloc &) {  // no host memory to remember it
+    size_.erase(it);
+    (void)hipFree(p);
+    return;
+  }
+  idle_bytes_ += it->second;
   give_back(kPoolBytes);
 }
 

@@ -117,3 +117,20 @@ def test_merge_windows_of_small_units(run):
         names = [c[2] for c in log() if c[0] == "launch"]
         assert any("k_merge_winILi13E" in k for k in names) and not any("k_merge_winILi11E" in k for k in names)
     """)
+
+
+def test_release_without_host_memory(run):
+    """Releasing a graph needs no host memory: no exception leaves the library,
+    and what the pool cannot note goes back to the device."""
+    run("""
+    with cn.Context(0) as ctx:
+        held = fake.fake_held()
+        rg = ctx.upload(edgeless(100000))
+        release, h = rg._lib.acc_graph_release, rg._h
+        rg._h = None
+        fake.fake_fail_new(0)
+        release(h)
+        fake.fake_fail_new(-1)
+        ctx.upload(edgeless(70000)).release()
+    assert fake.fake_held() == held == 0
+    """)
