@@ -780,7 +780,10 @@ int acc_cn_compute(acc_graph *g, int path, uint32_t flags) {
   // a lower slot that collects its edge's whole count starts at `plus`
   ACC_TRY(accfwd::launch_init(g, accfwd::lower_counts(g) ? plus : 0));
   ACC_TRY(record(g, timing, "k_init"));
-  ACC_TRY(accdense::launch_count(g));
+  if (g->dense.n_units) {
+    ACC_TRY(accdense::launch_count(g));
+    ACC_TRY(record(g, timing, "k_dense"));
+  }
   ACC_TRY(accfwd::launch_count(g));
   ACC_TRY(record(g, timing, ("k_fwd_count<" + std::to_string(g->fwd_unroll) + ">").c_str()));
   if (g->n_fwd_big) {
