@@ -196,7 +196,7 @@ void plan_dense(acc_graph *g, bool dense, std::vector<FwdUnit> &units, std::vect
     for (uint32_t b = lo; b < hi; b++) {
       p.max_low = std::max(p.max_low, hs[b] - off[b]);
       for (uint32_t j0 = hs[b]; j0 < off[b + 1]; j0 += g->chunk)
-        units.push_back(FwdUnit{static_cast<int32_t>(b), j0, std::min(j0 + g->chunk, off[b + 1]), v0});
+        units.push_back(FwdUnit{static_cast<int32_t>(b), j0, std::min(j0 + g->chunk, off[b + 1]), 0});
     }
   }
   if (at < g->shard_hi) rest.emplace_back(at, g->shard_hi);
@@ -971,8 +971,15 @@ int acc_tune(acc_graph *g, uint32_t flags, char *report, int report_cap) {
   for (const Axis &ax : axes) {
     int64_t keep = 0;
     ACC_TRY(acc_graph_get_param(g, ax.param, &keep));
+    std::vector<uint32_t> grids(1, accfwd::count_persist(g, g->persist));
     for (int64_t v : ax.values) {
       if (v == keep) continue;
+      // a grid that launches as one before it did is no trial (k_dense takes the parameter as it is)
+      if (ax.param == ACC_PARAM_PERSIST && !g->dense.n_units) {
+        const uint32_t grid = accfwd::count_persist(g, static_cast<uint32_t>(v));
+        if (std::find(grids.begin(), grids.end(), grid) != grids.end()) continue;
+        grids.push_back(grid);
+      }
       ACC_TRY(acc_graph_set_param(g, ax.param, v));
       float ms = 0;
       ACC_TRY(time_pass(g, ACC_PATH_FORWARD, reps, &ms));

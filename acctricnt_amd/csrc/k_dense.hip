@@ -22,7 +22,7 @@
 // row and column sums of c's hit matrix: k_dense_rows reads every matrix once
 // and adds them to c's lower slots, where an update of one 4-byte count per
 // triangle by a global atomic took most of the pass before.  The lower slots
-// then hold the complete counts and k_dense_gather copies them to the upper
+// then hold the complete counts and k_combine copies them to the upper
 // slots.  Matrices of vertices with more than hit_cap dense neighbors are not
 // kept (their size grows with the square), and none where the device has no
 // memory left for them; their probes update the counts by atomics.
@@ -303,7 +303,7 @@ static_assert(kDenseLdsBytes % 16 == 0, "the set is cleared in 16-byte steps, th
 // b with at most kChunk of its upper slots (b, c): the workgroup builds the
 // set of N<(b), lays the probes' 8-element groups end to end and gives every
 // lane one group per row of 64.  The U rows of a round are loaded while the
-// round before is decided.  u.nlow is the graph's first vertex.
+// round before is decided.
 template <int U, bool kSlots>
 __global__ __launch_bounds__(kWG, 8) void k_dense(const uint4 *__restrict__ vmeta, const int32_t *__restrict__ adj,
                                                   const uint32_t *__restrict__ rev, const uint4 *__restrict__ low,
@@ -472,14 +472,11 @@ __global__ __launch_bounds__(kWG, 8) void k_dense(const uint4 *__restrict__ vmet
 }
 
 // ---------------------------------------------------------------- hit matrices
-// Sum over the 2^log lanes of a group (consecutive lanes, log <= 6) in its last lane.
+// Sum over the 2^log lanes of a group (consecutive lanes, log <= 3: a tile's words) in its last lane.
 __device__ __forceinline__ uint32_t group_sum(uint32_t x, int log) {
   if (log > 0) x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
   if (log > 1) x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
   if (log > 2) x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
-  if (log > 3) x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
-  if (log > 4) x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-  if (log > 5) x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
   return x;
 }
 
@@ -541,6 +538,7 @@ struct ColumnSums {
 // 64 >> log rows a step, kTurns waves taking turns at the steps.  Row and column sums
 // are added to sums[] in LDS.
 constexpr uint32_t kTileWords = 8;
+static_assert(kTileWords <= 8, "group_sum adds groups of up to 8 lanes");
 template <uint32_t kTurns>
 __device__ __forceinline__ void sum_matrix(const uint8_t *__restrict__ H, uint32_t d, uint32_t *sums, int wave,
                                            int lane) {

@@ -1054,14 +1054,7 @@ int launch_count_t(acc_graph *g, unsigned long long *total) {
   hipStream_t st = g->ctx->stream;
   const bool to_lower = accfwd::lower_counts(g);
   const uint64_t tasks = g->n_fwd_block + (g->n_fwd_wave + kWaves - 1) / kWaves;
-  // A workgroup holds its place until the slowest of its waves has ended, so
-  // several tasks a workgroup even out unequal packs: at 64 workgroups per
-  // compute unit 512 packed graphs (average degree 22) took 5.60 ms against
-  // 6.03 at 256, Erdos-Renyi n = 2M, degree 26, 1.48 against 1.55, n = 3M,
-  // degree 40, 4.05 against 4.19.  Below an average degree of 16 packs are
-  // short and alike and the finer grid ends evenly: n = 8M, degree 8, 1.76 ms at
-  // 256 against 1.81 at 64; degrees 16 and 20 are within 1% either way.
-  const uint64_t per_cu = g->m >= 16ull * g->n ? std::min<uint32_t>(g->persist, 64) : g->persist;
+  const uint64_t per_cu = accfwd::count_persist(g, g->persist);
   const uint64_t cap = per_cu * static_cast<uint64_t>(g->ctx->num_cus);
   const unsigned grid = static_cast<unsigned>(g->persist && cap < tasks ? cap : tasks);
   if (grid) {
