@@ -28,12 +28,12 @@
 // memory left for them; their probes update the counts by atomics.
 //
 // Measured at R-MAT scale 22 (4.2M vertices, 128M slots, 94% of 7.2e9 probe
-// elements at dense sources): counting 4.4 ms + 1.1 ms for the other sources
+// elements at dense sources): counting 4.5 ms + 1.0 ms for the other sources
 // and 0.8 ms for the sums, where the other form took 17.1 ms for all; the
 // copy to the upper slots 1.25 ms against 2.2 ms for adding both; the whole
-// pass 20.0 to 7.7 ms.  The triangle-only pass, 6.1 to 3.3 ms, is bound by the
-// lists' traffic (16-bit ids halve it; 18 GB fetched), the per-slot counting by VALU (74%
-// busy) and LDS (58%); its hit bytes and (b, a) counters cost 0.8 ms each.
+// pass 20.0 to 7.6 ms.  The triangle-only pass, 6.1 to 3.3 ms, is bound by the
+// lists' traffic (16-bit ids halve it; 17.4 GB fetched), the per-slot counting by VALU (74%
+// busy) and LDS (59%); its hit bytes and (b, a) counters cost 0.8 ms each.
 
 #include <hip/hip_runtime.h>
 

@@ -252,7 +252,8 @@ int acc_scan_pairs(acc_scan_ws *ws, int32_t *pairs, uint64_t cap, uint64_t *coun
  * query per process, scan-query/scan_xp.cpp:2083-2110). */
 typedef struct acc_server acc_server;
 typedef struct acc_server_config {
-  uint64_t hbm_budget; /* device bytes for resident graphs plus result slots */
+  uint64_t hbm_budget; /* device bytes for resident graphs plus result slots, and what the context keeps
+                          of released graphs */
   int32_t max_batch;   /* queries per batched launch, 1..14 (the job table is a kernel argument) */
   int32_t streams;     /* batches in flight at once, 1..16 */
   int32_t slots;       /* queries holding results at once (launched, not released), 1..4096 */
